@@ -149,3 +149,48 @@ def test_many_row_form_vs_oracle(dqk):
     live = cnt > 0
     torch.testing.assert_close(res["lse"].cpu()[live], rl[live], atol=1e-3, rtol=1e-4)
     assert (res["lse"].cpu()[~live] < -1e29).all()
+
+
+@pytest.mark.parametrize("rows_form", [False, True])
+@pytest.mark.parametrize("dqk", [576, 512])
+def test_many_row_form_moving_maxima(dqk, rows_form):
+    """The many-row form on rows whose scores keep rising along the selection (kv scales growing 3,000-fold, so the
+    running maximum moves, and the output is rescaled, in most chunks), and falling (it moves once), with 128 heads,
+    pages of 48 (no power of two) and the rows + count form; bf16 outputs against the oracle. The bound is the file's
+    2e-2: the largest scale is 1, so a value is at most about 4.6, and the weights' rounding to bf16 (2^-9 of sum p |v|)
+    and the output's (2^-9 of it) are at most 0.009 each."""
+    g = torch.Generator().manual_seed(dqk + rows_form)
+    B, H, L, ps, keep = 130, 128, 480, 48, 448
+    say(f"attention many-row form, moving maxima dqk={dqk} rows={rows_form}")
+    npg = L // ps
+    num_pages = 1 + npg
+    kv = torch.randn(num_pages * ps, dqk, generator=g).to(W.FP8)
+    table = (torch.randperm(npg, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    up = torch.logspace(-3.5, 0.0, L)  # by position
+    scale_of = torch.ones(num_pages * ps)
+    slot = O.token_slots(table[0], torch.arange(L), ps)
+    scale_of[slot] = up
+    q = torch.randn(B, H, dqk, generator=g).to(torch.bfloat16)
+    cnt = torch.randint(1, keep + 1, (B,), generator=g)
+    cnt[:5] = torch.tensor([keep, 0, 1, 65, 128])
+    idx = torch.zeros(B, keep, dtype=torch.int64)
+    for b in range(B):
+        n = int(cnt[b])
+        idx[b, :n] = torch.randperm(L, generator=g)[:n].sort(descending=bool(b & 1)).values
+    if rows_form:
+        from trnrt_amd.kernels import dsa_slots_c
+        rows = torch.stack([O.token_slots(table[b], idx[b], ps) for b in range(B)])
+        bias = torch.where(torch.arange(keep).view(1, -1) < cnt.view(-1, 1), 0.0, -1e30)
+        o, lse = dsa_slots_c.attend(q.cuda(), kv.cuda(), rows.int().cuda(), bias.cuda(), 0.6, lse=True,
+                                    kc_scale=scale_of.cuda())
+        ro, rl = O.sparse_mla_ref(q, kv, scale_of, idx, cnt, table, ps, 0.6)
+        live = cnt > 0
+        o, ro = o[live.cuda()], ro[live]
+    else:
+        o, lse = dsa_decode.attend_tokens(q.cuda(), kv.cuda(), scale_of.cuda(), idx.cuda(), cnt.cuda(), table.cuda(),
+                                          ps, 0.6)
+        ro, rl = O.sparse_mla_ref(q, kv, scale_of, idx, cnt, table, ps, 0.6)
+        live = cnt > 0
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu()[live], rl[live], atol=1e-3, rtol=1e-4)
+    assert (lse.cpu()[~live] < -1e29).all()
