@@ -258,7 +258,8 @@ size_t dsa_prefill_select_workspace_bytes(int N, int P, int score_stride, int ke
  * scores/idx/cnt are the intermediates the caller may read afterwards (scores fp32 [B, score_stride], idx int32
  * [B, keep], cnt int32 [B]). On a GPU of 8 XCDs x 32 CUs with rows of at most 32,768 tokens (and the shapes the
  * one-launch kernel takes: Hi <= 64, H a multiple of 16 up to 512, pages of a power of two >= 32, score_stride a
- * multiple of 4, keep <= 256 * (512 / H)) the step is one kernel launch; otherwise it is dsa_decode_layer_chain.
+ * multiple of 4, keep <= 256 * (512 / H)) a step of at most 16 rows (any number with splits given) is one kernel launch
+ * per 8 rows; otherwise it is dsa_decode_layer_chain.
  * The one launch, and the separate kernels' attention launch, are 256 workgroups of which the 32 on each XCD wait
  * for each other at XCD-local barriers: they need every one of their workgroups resident at once (one per CU, 160
  * KiB of LDS each). So these calls must not overlap one another on a GPU, whatever their workspaces and streams,

@@ -151,6 +151,31 @@ def test_many_row_form_vs_oracle(dqk):
     assert (res["lse"].cpu()[~live] < -1e29).all()
 
 
+@pytest.mark.parametrize("B,H,keep", [(9, 64, 2048), (43, 64, 2048), (5, 128, 4160), (70, 64, 192), (140, 128, 64)])
+def test_many_row_form_in_splits(B, H, keep):
+    """The many-row form in splits (from 9 workgroups' rows on; 8, 5, 8, 3 and 1 of them here), counts that leave the
+    last splits empty (0, 1, one chunk, a chunk and one slot, all), against the oracle; slots of one 4,224-token context."""
+    g = torch.Generator().manual_seed(B + keep)
+    say(f"attention many-row form in splits B={B} H={H} keep={keep}")
+    L, ps = 4224, 64
+    kv, ks = W.quantize_rows(torch.randn(L + ps, 576, generator=g))
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    q = torch.randn(B, H, 576, generator=g).to(torch.bfloat16)
+    cnt = torch.randint(0, keep + 1, (B,), generator=g)
+    cnt[:5] = torch.tensor([0, 1, 64, min(65, keep), keep])
+    idx = torch.zeros(B, keep, dtype=torch.int64)
+    for b in range(B):
+        n = int(cnt[b])
+        idx[b, :n] = torch.randperm(L, generator=g)[:n].sort().values
+    o, lse = dsa_decode.attend_tokens(q.cuda(), kv.cuda(), ks.cuda(), idx.cuda(), cnt.cuda(), table.cuda(), ps,
+                                      192 ** -0.5)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, 192 ** -0.5)
+    live = cnt > 0
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu()[live], rl[live], atol=1e-3, rtol=1e-4)
+    assert (lse.cpu()[~live] < -1e29).all()
+
+
 @pytest.mark.parametrize("rows_form", [False, True])
 @pytest.mark.parametrize("dqk", [576, 512])
 def test_many_row_form_moving_maxima(dqk, rows_form):

@@ -198,6 +198,41 @@ def test_layer_long_tied_row_every_tile_read():
     _attention_check(inp, L)
 
 
+@pytest.mark.parametrize("H, lengths, attend", [
+    # 17 and 18 rows: past the 16 of the one-launch layer; the even indexer split past 8,192 tokens, a workgroup per 512
+    # positions below; empty, one-token and full-keep rows; 64 heads in 8 splits (17 rows), all in one row block
+    (64, [12000, 0, 1, 2047, 2048, 2049, 9000, 31, 33, 64, 4095, 100, 11999, 8192, 8193, 500, 7], "wide"),
+    (64, [4097, 0, 1, 2047, 2048, 2049, 4096, 31, 33, 64, 4095, 100, 3000, 8000, 8192, 500, 7, 8191], "wide"),
+    # 128 heads (two workgroups a row and split): the many-row attention from 5 rows on
+    (128, [6000, 0, 2500, 1, 5999], "wide"),
+    # 32 heads: the XCD-local attention launch over three rows an XCD
+    (32, [9000, 0, 1, 2047, 2048, 2049, 8999, 31, 33, 64, 4095, 100, 3000, 8193, 8192, 500, 7], "xcd"),
+])
+def test_layer_batch_of_many_rows(H, lengths, attend):
+    """Batches that take the separate kernels: every stage against the oracle, the selection bit-exact, the histograms
+    left zero for the next call (two steps on one workspace)."""
+    from tests._helpers import launched_kernels
+    say(f"layer batch of {len(lengths)} rows, H={H}")
+    cfg = W.Config("layer-batch", B=len(lengths), L=max(lengths), H=H, Hi=48)
+    inp = W.make_inputs(cfg, seed=71 + H, lengths=lengths)
+    g = inp.to("cuda")
+    L = _layer(g)
+    names = launched_kernels(lambda: L.step(g.q_idx, g.w_k, g.k_cache, g.k_scale, g.q, g.kv_cache, g.kv_scale, g.table,
+                                            g.ctx_len))
+    torch.cuda.synchronize()
+    assert names[-1 if attend == "xcd" else -2] == ("decode_attend_kernel" if attend == "xcd" else
+                                                    "sparse_mla_wide_kernel"), names
+    sc = L.scores.cpu()
+    ref = O.indexer_ref(inp.q_idx, inp.w_k, inp.k_cache, inp.k_scale, inp.table, inp.ctx_len, cfg.page_size,
+                        sc.shape[1])
+    assert row_rel_err(sc, ref, ref > -1e29) <= 1e-2
+    assert torch.all(sc[ref <= -1e29] < -1e29)
+    ri, rc = O.topk_ref(sc, cfg.keep, inp.ctx_len)
+    assert torch.equal(L.idx.cpu().long(), ri) and torch.equal(L.cnt.cpu().long(), rc)
+    _attention_check(inp, L)
+    assert L.status()["gave_up"] == 0
+
+
 def _sampled_indexer_check(g, sc, nsample=4096, seed=0):
     cfg = g.cfg
     gen = torch.Generator().manual_seed(seed)

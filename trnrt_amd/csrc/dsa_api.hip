@@ -101,7 +101,7 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
                              float* lse, void* ws, int B, int H, int Dqk, int keep, int max_pages, int page_size,
                              int num_pages, float scale, int splits, hipStream_t s, PoolForm pf = PoolForm{},
                              bool wide = false);
-bool attention_wide_ok(int B, int H, int keep, bool has_bias, int num_cu);
+int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int num_cu);
 hipError_t launch_token_rows(const int* idx, const int* cnt, const int* table, int* rows, float* bias, int B,
                              int keep, int max_pages, int page_size, int num_pages, hipStream_t s);
 int attention_default_splits(int B, int H, int keep, int num_cu);
@@ -151,6 +151,41 @@ int effective_splits(int splits, int keep) {
   int sps = (keep + splits - 1) / splits;
   sps = (sps + 63) / 64 * 64;
   return (keep + sps - 1) / sps;
+}
+
+// The attention of B rows over `keep` token slots (the pooled form: plus up to `tail` tail slots): the many-row form
+// over its splits, or the split form's effective split count.
+struct AttPlan {
+  bool wide;
+  int splits;
+};
+
+AttPlan attention_plan(int B, int H, int keep, int tail, bool has_bias, int splits) {
+  const int w = dsa::attention_wide_splits(B, H, keep + tail, has_bias, splits, num_cu());
+  if (w > 0) return {true, w};
+  return {false, effective_splits(resolve_splits(splits, B, H, keep), keep)};
+}
+
+// The larger of the workspaces of the two forms that a call may take (with a bias array or without).
+size_t attention_bytes(int B, int H, int keep, int tail, int splits) {
+  const AttPlan p = attention_plan(B, H, keep, tail, false, splits), q = attention_plan(B, H, keep, tail, true, splits);
+  const size_t a = dsa::attention_workspace_bytes(B, H, p.splits), b = dsa::attention_workspace_bytes(B, H, q.splits);
+  return a > b ? a : b;
+}
+
+// A decode batch of more rows than this takes the separate kernels even where the one-launch layer takes its shape: the
+// one launch handles 8 rows at a time, each a chain of latencies (about 25 us), where the separate kernels' grids share
+// the whole batch. Measured, 64 heads, rows of 500 to 32,768 tokens, one launch per 8 rows against the separate kernels:
+// 17 rows 73 and 45 us, 24 rows 75 and 52, 48 rows 151 and 71, 64 rows 215 and 85; rows of 4,096: 24 rows 69 and 39, 48
+// rows 137 and 49; 32 heads: 48 rows 145 and 92. (At 9 to 16 rows, two launches, they are 46-51 and 41-44.)
+constexpr int kBatchRows = 16;
+
+// The decode layer's attention within the workspace it is given: the many-row form in as many of its splits as fit.
+AttPlan layer_attention_plan(int B, int H, int keep, int splits, size_t bytes) {
+  AttPlan p = attention_plan(B, H, keep, 0, false, splits);
+  while (p.wide && p.splits > 1 && dsa::attention_workspace_bytes(B, H, p.splits) > bytes)
+    p.splits = effective_splits(p.splits - 1, keep);
+  return p;
 }
 
 // The prefill selection runs over tiles of T query rows: each tile's scores [T, score_stride] fp32, then its
@@ -645,16 +680,15 @@ static int sparse_mla_decode(const void* q_bf16, const uint8_t* kv_fp8, const fl
   if ((Dqk != 576 && Dqk != 512) || Dv != 512 || H % 16) return DSA_EUNSUPPORTED;
   if ((long)num_pages * page_size > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (B == 0) return DSA_OK;
-  const int sp = effective_splits(resolve_splits(splits, B, H, keep), keep);
-  const size_t need = dsa::attention_workspace_bytes(B, H, sp);
+  const AttPlan plan = attention_plan(B, H, keep, 0, bias != nullptr, splits);
+  const size_t need = dsa::attention_workspace_bytes(B, H, plan.splits);
   if (need && (!workspace || workspace_bytes < need)) return DSA_EWORKSPACE;
-  const bool wide = sp == 1 && dsa::attention_wide_ok(B, H, keep, bias != nullptr, num_cu()) && (token_form || cnt);
   dsa::PoolForm pf{};
   pf.n_live = n_live;
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, idx, cnt, page_table,
                                        rows, bias, static_cast<uint16_t*>(out_bf16), out_f32, lse, workspace, B, H,
-                                       Dqk, keep, max_pages, page_size, num_pages, scale, sp,
-                                       static_cast<hipStream_t>(stream), pf, wide));
+                                       Dqk, keep, max_pages, page_size, num_pages, scale, plan.splits,
+                                       static_cast<hipStream_t>(stream), pf, plan.wide));
 }
 
 extern "C" {
@@ -700,7 +734,7 @@ size_t dsa_slots_compact_workspace_bytes(int B, int H, int NS, int kp, int split
   if (B < 0 || H < 16 || NS < 1 || kp < 1) return 0;
   const int T = NS * kp;
   return align256((size_t)B * T * 4) + align256((size_t)B * 4) +
-         align256(dsa::attention_workspace_bytes(B, H, effective_splits(resolve_splits(splits, B, H, T), T)));
+         align256(dsa::attention_workspace_bytes(B, H, attention_plan(B, H, T, 0, false, splits).splits));
 }
 
 int dsa_sparse_mla_slots_compact(const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale,
@@ -723,13 +757,13 @@ int dsa_sparse_mla_slots_compact(const void* q_bf16, const uint8_t* kv_fp8, cons
   if (dsa::launch_compact_slots(rows, bias, B, NS, kp, (int)(num_slots / kp), tok, tcnt, s) != hipSuccess)
     return DSA_ELAUNCH;
   // the compacted rows + count form; a row with no visible token attends its list's kp entries, all masked
-  const int sp = effective_splits(resolve_splits(splits, B, H, T), T);
+  const AttPlan plan = attention_plan(B, H, T, 0, false, splits);
   dsa::PoolForm pf{};
   pf.empty_n = kp;
-  const bool wide = sp == 1 && dsa::attention_wide_ok(B, H, T, false, num_cu());
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, nullptr, tcnt,
                                        nullptr, tok, nullptr, static_cast<uint16_t*>(out_bf16), out_f32, lse, aws, B,
-                                       H, Dqk, T, 1, 1, (int)num_slots, scale, sp, s, pf, wide));
+                                       H, Dqk, T, 1, 1, (int)num_slots, scale, plan.splits, s, pf,
+                                       plan.wide));
 }
 
 int dsa_token_rows(const int32_t* idx, const int32_t* cnt, const int32_t* page_table, int32_t* rows, float* bias,
@@ -753,34 +787,41 @@ int dsa_pool_slots(const int32_t* pools, const int32_t* cnt, const int32_t* npoo
                                        n_slots, table_pages, page_size, kp, static_cast<hipStream_t>(stream)));
 }
 
+// The least workspace the decode layer runs in (the many-row attention then takes the splits that fit).
+static size_t layer_min_bytes(int B, int H, int keep, int max_len, int splits) {
+  const size_t t = align256(dsa::topk_workspace_bytes(B, max_len, keep)) + layer_rows_bytes(B, keep);
+  if (H < 16) return align256(t);
+  const int sp = effective_splits(resolve_splits(splits, B, H, keep), keep);
+  size_t total = align256(t) + align256(dsa::attention_workspace_bytes(B, H, sp));
+  // the one-launch layer's layout shares the zero region and needs its own rest; the separate kernels' XCD-local
+  // attention takes the attention's place
+  const size_t f = dsa::fused_layer_bytes(dsa::topk_zero_bytes(B), B, H, keep);
+  const size_t x = align256(t) + align256(dsa::attend_xcd_bytes(B, H, keep));
+  // rows past 32,768 tokens: the selection, attention and combine in one launch, its lists past the attention's
+  const size_t lg = align256(t) + align256(dsa::long_attend_bytes(B, H, keep, max_len));
+  total = f > total ? f : total;
+  total = x > total ? x : total;
+  return lg > total ? lg : total;
+}
+
 size_t dsa_workspace_bytes(int kind, int B, int H, int keep, int max_len, int splits) {
   if (B < 0 || keep < 1) return 0;
-  size_t t = 0, a = 0;
-  if (kind == DSA_WS_TOPK || kind == DSA_WS_LAYER) t = dsa::topk_workspace_bytes(B, max_len, keep);
-  if (kind == DSA_WS_LAYER) t = align256(t) + layer_rows_bytes(B, keep);
-  if (kind == DSA_WS_ATTENTION || kind == DSA_WS_LAYER) {
-    if (H < 16) return align256(t);
-    const int sp = effective_splits(resolve_splits(splits, B, H, keep), keep);
-    a = dsa::attention_workspace_bytes(B, H, sp);
-  }
-  size_t total = align256(t) + align256(a);
-  if (kind == DSA_WS_LAYER) {
-    // the one-launch layer's layout shares the zero region and needs its own rest; the separate kernels' XCD-local
-    // attention takes the attention's place
-    const size_t f = dsa::fused_layer_bytes(dsa::topk_zero_bytes(B), B, H, keep);
-    const size_t x = align256(t) + align256(dsa::attend_xcd_bytes(B, H, keep));
-    // rows past 32,768 tokens: the selection, attention and combine in one launch, its lists past the attention's
-    const size_t lg = align256(t) + align256(dsa::long_attend_bytes(B, H, keep, max_len));
-    total = f > total ? f : total;
-    total = x > total ? x : total;
-    total = lg > total ? lg : total;
+  if (kind == DSA_WS_TOPK) return align256(dsa::topk_workspace_bytes(B, max_len, keep));
+  if (kind == DSA_WS_ATTENTION) return H < 16 ? 0 : align256(attention_bytes(B, H, keep, 0, splits));
+  if (kind != DSA_WS_LAYER) return 0;
+  size_t total = layer_min_bytes(B, H, keep, max_len, splits);
+  const AttPlan p = H < 16 ? AttPlan{false, 1} : attention_plan(B, H, keep, 0, false, splits);
+  if (p.wide) {
+    const size_t w = align256(dsa::topk_workspace_bytes(B, max_len, keep)) + layer_rows_bytes(B, keep) +
+                     align256(dsa::attention_workspace_bytes(B, H, p.splits));
+    total = w > total ? w : total;
   }
   return total;
 }
 
 int dsa_default_splits(int B, int H, int keep) {
   if (B < 1 || H < 16 || keep < 1) return 1;
-  return effective_splits(resolve_splits(0, B, H, keep), keep);
+  return attention_plan(B, H, keep, 0, false, 0).splits;
 }
 
 static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
@@ -816,6 +857,31 @@ static int layer_checks(const void* q_idx_bf16, const float* w, const uint8_t* k
   return DSA_OK;
 }
 
+// The decode layer after its checks: in one launch where the shapes allow and the rows are few (kBatchRows), otherwise
+// the separate kernels.
+static int decode_layer(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
+                        const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale, const int32_t* page_table,
+                        const int32_t* ctx_len, float* scores, int32_t* idx, int32_t* cnt, void* out_bf16, float* lse,
+                        void* workspace, size_t workspace_bytes, int B, int Hi, int H, int max_pages, int page_size,
+                        int num_pages, int score_stride, int max_len, int keep, float scale, int splits,
+                        void* stream) {
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (ready_zero(workspace, dsa::topk_zero_bytes(B), s) != hipSuccess) return DSA_ELAUNCH;
+  const bool one = dsa::fused_layer_ok(num_cu(), Hi, H, max_len, keep, page_size, score_stride) &&
+                   (B <= kBatchRows || splits != 0);
+  const int r =
+      one ? status(dsa::launch_decode_fused(
+                static_cast<const uint16_t*>(q_idx_bf16), w, k_fp8, k_scale, static_cast<const uint16_t*>(q_bf16),
+                kv_fp8, kv_scale, page_table, ctx_len, scores, idx, cnt, static_cast<uint16_t*>(out_bf16), lse,
+                workspace, dsa::topk_zero_bytes(B), B, Hi, H, max_pages, page_size, num_pages, score_stride, keep,
+                scale, s))
+          : layer_chain(q_idx_bf16, w, k_fp8, k_scale, q_bf16, kv_fp8, kv_scale, page_table, ctx_len, scores, idx,
+                        cnt, out_bf16, lse, workspace, workspace_bytes, B, Hi, H, max_pages, page_size, num_pages,
+                        score_stride, max_len, keep, scale, splits, stream);
+  if (r != DSA_OK) drop_zero(workspace);
+  return r;
+}
+
 int dsa_decode_layer(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
                      const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale, const int32_t* page_table,
                      const int32_t* ctx_len, float* scores, int32_t* idx, int32_t* cnt, void* out_bf16, float* lse,
@@ -825,18 +891,9 @@ int dsa_decode_layer(const void* q_idx_bf16, const float* w, const uint8_t* k_fp
                               idx, cnt, out_bf16, workspace, workspace_bytes, B, Hi, H, max_pages, page_size,
                               num_pages, score_stride, max_len, keep, splits);
   if (st != DSA_OK || B == 0) return st;
-  if (!dsa::fused_layer_ok(num_cu(), Hi, H, max_len, keep, page_size, score_stride))
-    return dsa_decode_layer_chain(q_idx_bf16, w, k_fp8, k_scale, q_bf16, kv_fp8, kv_scale, page_table, ctx_len,
-                                  scores, idx, cnt, out_bf16, lse, workspace, workspace_bytes, B, Hi, H, max_pages,
-                                  page_size, num_pages, score_stride, max_len, keep, scale, splits, stream);
-  const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (ready_zero(workspace, dsa::topk_zero_bytes(B), s) != hipSuccess) return DSA_ELAUNCH;
-  const int r = status(dsa::launch_decode_fused(
-      static_cast<const uint16_t*>(q_idx_bf16), w, k_fp8, k_scale, static_cast<const uint16_t*>(q_bf16), kv_fp8,
-      kv_scale, page_table, ctx_len, scores, idx, cnt, static_cast<uint16_t*>(out_bf16), lse, workspace,
-      dsa::topk_zero_bytes(B), B, Hi, H, max_pages, page_size, num_pages, score_stride, keep, scale, s));
-  if (r != DSA_OK) drop_zero(workspace);
-  return r;
+  return decode_layer(q_idx_bf16, w, k_fp8, k_scale, q_bf16, kv_fp8, kv_scale, page_table, ctx_len, scores, idx, cnt,
+                      out_bf16, lse, workspace, workspace_bytes, B, Hi, H, max_pages, page_size, num_pages,
+                      score_stride, max_len, keep, scale, splits, stream);
 }
 
 int dsa_decode_layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
@@ -884,7 +941,11 @@ static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_
   char* lws = static_cast<char*>(workspace) + t_need + layer_rows_bytes(B, keep);
   float* tmax = la && dsa::long_attend_tiles(max_len) ? dsa::long_attend_tmax(lws, B, H, keep, max_len) : nullptr;
   hipError_t e;
-  if (flat)
+  // flat rows of a batch: the long rows' indexer too, whose workgroups share the batch's live tiles evenly whatever the
+  // rows' lengths (48 rows of 500 to 32,768 tokens 97 us a step with it, 114 with a workgroup per 512 positions of the
+  // longest row's; 48 rows of 4,096: 51 and 49)
+  const bool even = !flat || (B > kBatchRows && max_len > 8192);
+  if (!even)
     e = dsa::launch_indexer_decode(static_cast<const uint16_t*>(q_idx_bf16), w, k_fp8, k_scale, page_table, ctx_len,
                                    nullptr, scores, hist, B, Hi, max_pages, page_size, num_pages, score_stride,
                                    num_cu(), s);
@@ -925,21 +986,19 @@ static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_
   }
   char* aws = static_cast<char*>(workspace) + t_need + layer_rows_bytes(B, keep);
   const size_t aws_bytes = workspace_bytes - t_need - layer_rows_bytes(B, keep);
-  // the default split count on a GPU of 8 XCDs x 32 CUs: the one-launch layer's attention and combine as a launch of
-  // their own (XCD-local, bf16 split outputs), over the slot rows (flat rows) or the positions through the page table
-  if (splits == 0 && dsa::attend_xcd_ok(num_cu(), H, keep))
+  const AttPlan plan = layer_attention_plan(B, H, keep, splits, aws_bytes);
+  // the default split count on a GPU of 8 XCDs x 32 CUs, a batch of few rows (or head counts the many-row form does not
+  // take): the one-launch layer's attention and combine as a launch of their own (XCD-local, bf16 split outputs),
+  // over the slot rows (flat rows) or the positions through the page table
+  if (splits == 0 && dsa::attend_xcd_ok(num_cu(), H, keep) && !(plan.wide && B > kBatchRows))
     return status(dsa::launch_decode_attend(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, rows,
                                             rows ? nullptr : idx, page_table, cnt, static_cast<uint16_t*>(out_bf16),
                                             lse, aws, static_cast<int*>(workspace), B, H, max_pages, page_size,
                                             num_pages, keep, scale, s));
-  if (!rows)
-    return dsa_sparse_mla_decode(q_bf16, kv_fp8, kv_scale, idx, cnt, page_table, nullptr, nullptr, out_bf16, nullptr,
-                                 lse, aws, aws_bytes, B, H, 576, 512, keep, max_pages, page_size, num_pages, scale,
-                                 splits, stream);
-  const int sp = effective_splits(resolve_splits(splits, B, H, keep), keep);
-  return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, nullptr, cnt, nullptr,
-                                       rows, nullptr, static_cast<uint16_t*>(out_bf16), nullptr, lse, aws, B, H, 576,
-                                       keep, max_pages, page_size, num_pages, scale, sp, s));
+  return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, rows ? nullptr : idx,
+                                       cnt, rows ? nullptr : page_table, rows, nullptr,
+                                       static_cast<uint16_t*>(out_bf16), nullptr, lse, aws, B, H, 576, keep, max_pages,
+                                       page_size, num_pages, scale, plan.splits, s, dsa::PoolForm{}, plan.wide));
 }
 
 extern "C" {
@@ -956,21 +1015,21 @@ int dsa_decode_layer_noalloc(const void* q_idx_bf16, const float* w, const uint8
                               idx, cnt, out_bf16, nullptr, 0, B, Hi, H, max_pages, page_size, num_pages, score_stride,
                               max_len, keep, splits, false);
   if (st != DSA_OK) return st;
-  const size_t need = dsa_workspace_bytes(DSA_WS_LAYER, B, H, keep, max_len, splits);
+  const size_t need = layer_min_bytes(B, H, keep, max_len, splits);
   if (need == 0 || need > DSA_NOALLOC_SCRATCH_BYTES) return DSA_ESCRATCH;
   if (B == 0) return DSA_OK;
   void* ws = noalloc_scratch();
   if (!ws) return DSA_ELAUNCH;
-  return dsa_decode_layer(q_idx_bf16, w, k_fp8, k_scale, q_bf16, kv_fp8, kv_scale, page_table, ctx_len, scores, idx,
-                          cnt, out_bf16, lse, ws, DSA_NOALLOC_SCRATCH_BYTES, B, Hi, H, max_pages, page_size,
-                          num_pages, score_stride, max_len, keep, scale, splits, stream);
+  return decode_layer(q_idx_bf16, w, k_fp8, k_scale, q_bf16, kv_fp8, kv_scale, page_table, ctx_len, scores, idx, cnt,
+                      out_bf16, lse, ws, DSA_NOALLOC_SCRATCH_BYTES, B, Hi, H, max_pages, page_size, num_pages,
+                      score_stride, max_len, keep, scale, splits, stream);
 }
 
 size_t dsa_sparse_mla_pooled_workspace_bytes(int B, int H, int keep, int kp, int splits) {
   if (B < 0 || H < 16 || keep < 1 || kp < 2) return 0;
   const int keep_sel = kp * keep;  // the selected pools' token slots; the tail comes on top
-  return align256(dsa::attention_workspace_bytes(B, H, effective_splits(resolve_splits(splits, B, H, keep_sel),
-                                                                          keep_sel)));
+  return align256(
+      dsa::attention_workspace_bytes(B, H, attention_plan(B, H, keep_sel, kp, false, splits).splits));
 }
 
 int dsa_sparse_mla_pooled(const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale, const int32_t* pools,
@@ -986,15 +1045,14 @@ int dsa_sparse_mla_pooled(const void* q_bf16, const uint8_t* kv_fp8, const float
   if ((long)num_pages * page_size > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (B == 0) return DSA_OK;
   const int keep_sel = kp * keep;  // the selected pools' token slots; the tail comes on top
-  const int sp = effective_splits(resolve_splits(splits, B, H, keep_sel), keep_sel);
-  const size_t need = dsa::attention_workspace_bytes(B, H, sp);
+  const AttPlan plan = attention_plan(B, H, keep_sel, kp, false, splits);
+  const size_t need = dsa::attention_workspace_bytes(B, H, plan.splits);
   if (need && (!workspace || workspace_bytes < need)) return DSA_EWORKSPACE;
   const dsa::PoolForm pf = {__builtin_ctz((unsigned)kp), keep, npool, positions, 0, 0, nullptr};
-  const bool wide = sp == 1 && dsa::attention_wide_ok(B, H, keep_sel + kp, false, num_cu());
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, pools, cnt, page_table,
                                        nullptr, nullptr, static_cast<uint16_t*>(out_bf16), out_f32, lse, workspace, B,
-                                       H, Dqk, keep_sel, max_pages, page_size, num_pages, scale, sp,
-                                       static_cast<hipStream_t>(stream), pf, wide));
+                                       H, Dqk, keep_sel, max_pages, page_size, num_pages, scale, plan.splits,
+                                       static_cast<hipStream_t>(stream), pf, plan.wide));
 }
 
 size_t dsa_pooled_workspace_bytes(int B, int H, int keep, int max_len, int kp, int splits) {

@@ -533,6 +533,19 @@ size_t attention_workspace_bytes(int B, int H, int splits) {
   return (size_t)B * splits * H * ATT_DV * 4 + (size_t)B * splits * H * 8 + 256;
 }
 
+static hipError_t combine(const float* ws_o, const float* ws_ml, int B, int H, int splits, uint16_t* out,
+                          float* out_f32, float* lse, const int* n_live, hipStream_t s) {
+  const dim3 grid(B * H), block(128);
+  if (splits <= 8)
+    return launch("combine_splits_kernel", combine_splits_kernel<8>, grid, block, s, ws_o, ws_ml, H, splits, out,
+                  out_f32, lse, n_live);
+  if (splits <= 16)
+    return launch("combine_splits_kernel", combine_splits_kernel<16>, grid, block, s, ws_o, ws_ml, H, splits, out,
+                  out_f32, lse, n_live);
+  return launch("combine_splits_kernel", combine_splits_kernel<32>, grid, block, s, ws_o, ws_ml, H, splits, out,
+                out_f32, lse, n_live);
+}
+
 hipError_t launch_sparse_mla_wide(const uint16_t* q, const uint8_t* kv, const float* kvs, const int* idx,
                                   const int* cnt, const int* table, const int* rows, uint16_t* out, float* out_f32,
                                   float* lse, float* ws_o, float* ws_ml, int B, int H, int Dqk, int keep,
@@ -545,12 +558,18 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
                              const int* table, const int* rows, const float* bias, uint16_t* out, float* out_f32,
                              float* lse, void* ws, int B, int H, int Dqk, int keep, int max_pages, int page_size,
                              int num_pages, float scale, int splits, hipStream_t s, PoolForm pf, bool wide) {
-  if (splits == 1 && wide) {
+  if (wide) {
     // the many-row form takes the pooled tail among its slots: kpool more
-    const int keep_w = pf.kp_shift ? keep + (1 << pf.kp_shift) : keep;
+    if (pf.kp_shift) keep += 1 << pf.kp_shift;
     pf.tail_apart = 0;
-    return launch_sparse_mla_wide(q, kv, kvs, idx, cnt, table, rows, out, out_f32, lse, nullptr, nullptr, B, H, Dqk,
-                                  keep_w, max_pages, page_size, num_pages, scale, 1, keep_w, pf, s);
+    const int sps = ((keep + splits - 1) / splits + ATT_CH - 1) / ATT_CH * ATT_CH;
+    const int eff = (keep + sps - 1) / sps;
+    float* ws_o = eff > 1 ? static_cast<float*>(ws) : nullptr;
+    float* ws_ml = eff > 1 ? ws_o + (size_t)B * eff * H * ATT_DV : nullptr;
+    const hipError_t e = launch_sparse_mla_wide(q, kv, kvs, idx, cnt, table, rows, eff > 1 ? nullptr : out,
+                                                eff > 1 ? nullptr : out_f32, lse, ws_o, ws_ml, B, H, Dqk, keep,
+                                                max_pages, page_size, num_pages, scale, eff, sps, pf, s);
+    return e != hipSuccess || eff == 1 ? e : combine(ws_o, ws_ml, B, H, eff, out, out_f32, lse, pf.n_live, s);
   }
   // the split form adds the pooled tail apart from its keep slots when its rows fit their LDS (kpool 8 with 576-wide
   // rows: 7 x 576 bytes do not; the tail is then among the slots, keep + kpool of them)
@@ -577,15 +596,8 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
           : launch("sparse_mla_kernel", sparse_mla_kernel<576>, dim3(grid), dim3(ATT_THREADS), s, q, kv, kvs, idx, cnt,
                    table, rows, bias, out, out_f32, lse, ws_o, ws_ml, B, H, keep, max_pages, page_size, num_pages,
                    scale, eff_splits, sps, pf);
-  if (e != hipSuccess || eff_splits == 1) return e;
-  if (eff_splits <= 8)
-    return launch("combine_splits_kernel", combine_splits_kernel<8>, dim3(B * H), dim3(128), s, ws_o, ws_ml, H,
-                  eff_splits, out, out_f32, lse, pf.n_live);
-  if (eff_splits <= 16)
-    return launch("combine_splits_kernel", combine_splits_kernel<16>, dim3(B * H), dim3(128), s, ws_o, ws_ml, H,
-                  eff_splits, out, out_f32, lse, pf.n_live);
-  return launch("combine_splits_kernel", combine_splits_kernel<32>, dim3(B * H), dim3(128), s, ws_o, ws_ml, H,
-                eff_splits, out, out_f32, lse, pf.n_live);
+  return e != hipSuccess || eff_splits == 1 ? e
+                                             : combine(ws_o, ws_ml, B, H, eff_splits, out, out_f32, lse, pf.n_live, s);
 }
 
 hipError_t launch_token_rows(const int* idx, const int* cnt, const int* table, int* rows, float* bias, int B,

@@ -472,10 +472,22 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
   }
 }
 
-// Whether a launch takes this form: 64-head workgroups, the token form or rows + cnt (no bias array), at most
-// AW_MAXSLOTS slots, and at least one workgroup per CU.
-bool attention_wide_ok(int B, int H, int keep, bool has_bias, int num_cu) {
-  return H % AW_HEADS == 0 && keep <= AW_MAXSLOTS && !has_bias && (long)B * (H / AW_HEADS) >= num_cu;
+// The splits this form takes a launch of B rows in, or 0 when it does not take it: 64-head workgroups, the token form
+// or rows + cnt (no bias array), at most AW_MAXSLOTS slots a split. An asked split count of 1 takes it when the rows
+// fill the GPU. Left to the library (splits 0), every launch of more than 8 workgroups' rows takes it, in as many
+// splits as keep one workgroup a CU, at most 8 (256 slots at keep 2,048: past that the fp32 split outputs cost what the
+// shorter splits gain). Measured against the split form (16 heads a workgroup), 2,048 slots of 576 bytes, attention
+// with its combine, 64 heads: 8 rows 21.5 us there and 21.9 here, 12 rows 37.7 and 22.8, 16 rows 27.4 and 23.0, 48
+// rows 70.8 and 32.7, 96 rows 125 and 47, 192 rows 219 and 63; 128 heads: 12 rows 51 and 25.5, 48 rows 116 and 45.
+int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int num_cu) {
+  if (B < 1 || H < AW_HEADS || H % AW_HEADS || has_bias || keep < 1 || splits > 1) return 0;
+  const long units = (long)B * (H / AW_HEADS);
+  if (splits == 1) return keep <= AW_MAXSLOTS && units >= num_cu ? 1 : 0;
+  if (units <= 8) return 0;
+  long s = num_cu / units;
+  s = s < 1 ? 1 : s > 8 ? 8 : s;
+  const int sps = (int)((keep + s - 1) / s + AW_CH - 1) / AW_CH * AW_CH;
+  return sps <= AW_MAXSLOTS ? (keep + sps - 1) / sps : 0;
 }
 
 hipError_t launch_sparse_mla_wide(const uint16_t* q, const uint8_t* kv, const float* kvs, const int* idx,

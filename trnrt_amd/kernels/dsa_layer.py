@@ -1,7 +1,7 @@
 """One DSA decode layer step on gfx950 in one call: indexer -> top-k -> sparse MLA, the order of
 trnrt/models/mla.py:506-528 `attention_long` (at kpool 1, with the q_lat / W_UV projections outside, as there). For
-rows of up to 32,768 tokens the step is one kernel launch (csrc/dsa_fused.hip); otherwise, or with chain=True, the
-separate kernels enqueued back to back.
+up to 16 rows of up to 32,768 tokens the step is one kernel launch per 8 rows (csrc/dsa_fused.hip); otherwise, or with
+chain=True, the separate kernels enqueued back to back.
 
 DecodeLayer preallocates the intermediates (scores, indices, counts) and the workspace once for a batch shape, so a
 step allocates nothing and can be captured in a HIP graph; step() enqueues the three operators on the current stream
