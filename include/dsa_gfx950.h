@@ -336,7 +336,7 @@ size_t dsa_sparse_mla_pooled_workspace_bytes(int B, int H, int keep, int kp, int
  *   before first use (calls leave the regions that must start at zero at zero). kp a power of two in [2, 8] dividing
  *   page_size; Hi <= 64; H a multiple of 16; Dqk 512 or 576. On a GPU of 8 XCDs x 32 CUs, with splits 0, Dqk 512,
  *   Hi <= 32, rows of at most 8,192 pools (max_pages page_size / kp, a multiple of 4), pages of at least 16 pools
- *   and keep kp <= 4096 / (H / 32) (H a multiple of 32), the step is one kernel launch per 8 rows (the indexer,
+ *   and keep kp <= 4096 / (H / 32) (H a multiple of 32), a step of at most 16 rows is one kernel launch per 8 (the indexer,
  *   the selection, the attention and the combine; XCD-local barriers, as dsa_decode_layer's one launch: the same
  *   co-residency rule and status words). Otherwise it is dsa_pooled_decode_layer_chain.
  */

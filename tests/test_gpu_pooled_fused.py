@@ -101,6 +101,21 @@ def test_pooled_fused_tails_and_short_rows(H):
     _check(cfg, inp, f, pos, npool)
 
 
+@pytest.mark.parametrize("H", [64, 32])
+def test_pooled_batch_of_many_rows(H):
+    """17 rows, past the 16 of the one launch: the separate kernels, with the many-row attention in splits at 64 heads
+    (the pooled token form: every tail length, a row with no complete pool, rows of fewer pools than keep, splits with no
+    slot) and the XCD-local launch at 32; against the oracle."""
+    positions = [8191, 8190, 8189, 8188, 4097, 2050, 2048, 2047, 700, 0, 1, 2, 3, 515, 1023, 6000, 3333]
+    cfg, inp, pos, npool = _inputs(len(positions), 8192, positions, H=H, seed=64 + H)
+    say(f"pooled batch of {len(positions)} rows H={H}")
+    layer = _layer(cfg, inp)
+    names = launched_kernels(lambda: _step(layer, inp, npool.cuda(), pos.cuda()))
+    assert ("sparse_mla_wide_kernel" if H == 64 else "decode_attend_kernel") in names, names
+    torch.cuda.synchronize()
+    _check(cfg, inp, layer, pos, npool)
+
+
 def test_pooled_fused_two_launches():
     """12 rows (two launches of 8 and 4 rows on one workspace), random positions in a 16,384-token context."""
     g = torch.Generator().manual_seed(63)

@@ -1065,7 +1065,10 @@ size_t dsa_pooled_workspace_bytes(int B, int H, int keep, int max_len, int kp, i
   const size_t x = align256(dsa::attend_xcd_bytes(B, H, keep_sel));
   // the one-launch form's layout shares the zero region and needs its own rest (key lists, split outputs)
   const size_t f = align256(dsa::fused_pooled_bytes(dsa::topk_zero_bytes(B), B, H));
-  const size_t chain = t + (a > x ? a : x);
+  const size_t w =
+      align256(dsa::attention_workspace_bytes(B, H, attention_plan(B, H, keep_sel, kp, false, splits).splits));
+  size_t chain = t + (a > x ? a : x);
+  chain = t + w > chain ? t + w : chain;
   return f > chain ? f : chain;
 }
 
@@ -1104,7 +1107,8 @@ static int pooled_layer_or_step(const void* q_idx_bf16, const float* w, const vo
                                pools, cnt, out_bf16, workspace, workspace_bytes, B, Hi, H, Dqk, max_pages, page_size,
                                num_pages, kp, keep, splits, &stride);
   if (st != DSA_OK || B == 0) return st;
-  if (splits != 0 || !dsa::fused_pooled_ok(num_cu(), Hi, H, Dqk, stride, kp, page_size, keep)) {
+  if (splits != 0 || B > kBatchRows ||
+      !dsa::fused_pooled_ok(num_cu(), Hi, H, Dqk, stride, kp, page_size, keep)) {
     if (pkw) {
       const int r = dsa_pool_keys_write(pkw->rows, pkw->rows_fp8, pkw->rows_scale, pkw->rows_width, pkw->ape,
                                         positions, page_table, 0, max_pages, pkw->slot_mapping,
@@ -1209,16 +1213,16 @@ static int pooled_layer(const void* q_idx_bf16, const float* w, const void* pool
   const int keep_sel = kp * keep;  // the selected pools' token slots; the tail comes on top
   // the default split count on a GPU of 8 XCDs x 32 CUs, 512-wide rows: the attention and combine in one XCD-local
   // launch (the separate kernels' form of the one-launch layer's last stages), the tail in the split of the last
-  // selected token; the barrier words are the workspace's first bytes
-  if (splits == 0 && dsa::attend_xcd_pooled_ok(num_cu(), H, Dqk, keep_sel))
+  // selected token; the barrier words are the workspace's first bytes (a batch of many rows: the many-row form)
+  const AttPlan plan = attention_plan(B, H, keep_sel, kp, false, splits);
+  if (splits == 0 && dsa::attend_xcd_pooled_ok(num_cu(), H, Dqk, keep_sel) && !(plan.wide && B > kBatchRows))
     return status(dsa::launch_decode_attend_pooled(
         static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, pools, cnt, npool, positions, page_table,
         static_cast<uint16_t*>(out_bf16), lse, static_cast<char*>(workspace) + t_need, static_cast<int*>(workspace), B,
         H, max_pages, page_size, num_pages, keep, __builtin_ctz((unsigned)kp), scale, s));
-  const int sp = effective_splits(resolve_splits(splits, B, H, keep_sel), keep_sel);
   const dsa::PoolForm pf = {__builtin_ctz((unsigned)kp), keep, npool, positions, 0, 0, nullptr};
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, pools, cnt, page_table,
                                        nullptr, nullptr, static_cast<uint16_t*>(out_bf16), nullptr, lse,
                                        static_cast<char*>(workspace) + t_need, B, H, Dqk, keep_sel, max_pages,
-                                       page_size, num_pages, scale, sp, s, pf));
+                                       page_size, num_pages, scale, plan.splits, s, pf, plan.wide));
 }
