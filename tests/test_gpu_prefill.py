@@ -74,6 +74,26 @@ def test_scores_fp8_queries_vs_oracle(N, Hi, P, stride):
     _check_scores(q8, w, k8, ks, npool, 128 ** -0.5, stride, qI_scale=qs, q_values=qv)
 
 
+@pytest.mark.parametrize("N,Hi,P,stride,high", [(3, 64, 9001, None, 300), (6, 64, 9001, 9004, 2177),
+                                                (5, 32, 6200, 6501, 2049), (2, 5, 33, 35, 33),
+                                                (9, 64, 4200, None, 128)])
+def test_scores_fp8_queries_candidates_end_early(N, Hi, P, stride, high):
+    """Workgroups stop at their queries' last candidate: inside a block's first round of 128 keys, at its edge, in a
+    later block, with rows that no 16-byte store fits; every other position is NEG_INF, and the rows round them are not
+    written. The bound is the file's (the products are exact, the sums in fp32)."""
+    say(f"prefill scores fp8 q N={N} Hi={Hi} P={P} stride={stride} candidates to {high}")
+    npool = torch.tensor([high, 0, 1, high - 1, 129, 32, 31, 127, 128][:N]).clamp(0, high)
+    qI, w, k8, ks, npool = _inputs(N, Hi, P, seed=N + P, npool=npool)
+    q8, qs, qv = _fp8(qI)
+    _check_scores(q8, w, k8, ks, npool, 128 ** -0.5, stride, qI_scale=qs, q_values=qv)
+    width = stride or P
+    buf = torch.full((N + 2, width), 7.0, device="cuda")
+    LS.scores(q8.cuda(), w.cuda(), k8.cuda(), npool.cuda(), 128 ** -0.5, pk_scale=ks.cuda(), stride=stride,
+              qI_scale=qs.cuda(), out=buf[1:-1])
+    torch.cuda.synchronize()
+    assert torch.all(buf[0] == 7.0) and torch.all(buf[-1] == 7.0)
+
+
 def test_fp8_query_argument_checks():
     qI, w, k8, ks, npool = _inputs(2, 8, 64, seed=1)
     q8, qs, _ = _fp8(qI)

@@ -28,9 +28,9 @@ constexpr int PF_QPW = PF_THREADS / WAVE;  // queries per workgroup
 constexpr int PF_TILES = 64;               // tiles per workgroup: 2048 keys
 constexpr int PF_TPB = 4;                  // tiles per barrier (a "round": 128 keys)
 constexpr int PF_RING = 2 * PF_TPB;        // tiles in flight per thread: two rounds ahead
-constexpr int PF8_TPB = 2;                 // rounds of 64 keys (fewer registers and LDS: 3 workgroups a CU)
-constexpr int PF8_RING = 2 * PF8_TPB;
-static_assert(PF_TILES % PF8_RING == 0, "a block is whole ring turns");
+constexpr int PF_TPB1 = 2;                 // at up to 32 heads
+constexpr int PF8_TPB = 4;                 // the FP8-query form's
+static_assert(PF_TILES % PF8_TPB == 0, "a block is whole rounds");
 static_assert(PF_TILES % PF_RING == 0, "a block is whole ring turns");
 
 // MT: head tiles of 32 (Hi <= 32 MT).
@@ -61,6 +61,20 @@ __device__ __forceinline__ void block_max_rows(const float* srow, int base, floa
   }
 }
 
+// A query's head weights (ws: one per head, 0 past its heads) in the accumulator layout: register r of head tile m holds
+// head 32 m + 8 (r / 4) + 4 h + r % 4.
+template <int MT>
+__device__ __forceinline__ void head_weights(const float* ws, int h, float (&wr)[MT][16]) {
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(ws + 32 * m + 8 * g + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wr[m][4 * g + e] = x[e];
+    }
+}
+
 // BF16K: the keys are bf16 [P, 128] with no per-key scale (GLM's pool keys, trnrt/models/dsa_long.py:74-84 over
 // trnrt/models/mla.py:491-503 `context_pool_keys`): a thread's share of a tile is 32 bytes (two loads) that go to
 // LDS as they are, so the ring holds twice the registers (taken at MT 1 only).
@@ -72,13 +86,14 @@ __global__ __launch_bounds__(PF_THREADS, MT == 1 ? 3 : 2) void indexer_prefill_k
   static_assert(!BF16K || MT == 1, "bf16 keys: up to 32 heads");
   // rounds of TPB tiles, RING in flight: at 32 heads rounds of 2 (fewer registers and LDS: 3 workgroups a CU), at 64
   // rounds of 4 (2 workgroups a CU; rounds of 2 there spill)
-  constexpr int TPB = MT == 1 ? PF8_TPB : PF_TPB, RING = 2 * TPB;
+  constexpr int TPB = MT == 1 ? PF_TPB1 : PF_TPB, RING = 2 * TPB;
   static_assert(PF_TILES % RING == 0, "a block is whole ring turns");
   const uint8_t* kcache = static_cast<const uint8_t*>(kcache_v);
   // two rounds of bf16 tiles (key j of a tile: 16 pieces of 8 dims, piece p at slot 16 j + (p ^ (j & 15))), the
   // block's per-key scales and the queries' candidate counts
   __shared__ u32x4 kb[2][TPB][PF_TILE * 16];
   __shared__ float ksc_s[PF_TILES * PF_TILE];
+  alignas(16) __shared__ float wsum[PF_QPW][WAVE];  // each query's head weights
   __shared__ int lmax[PF_QPW];
   const int wave = threadIdx.x / WAVE;
   const int lane = threadIdx.x & (WAVE - 1);
@@ -114,8 +129,7 @@ __global__ __launch_bounds__(PF_THREADS, MT == 1 ? 3 : 2) void indexer_prefill_k
   int L = min(max(npool[nq], 0), P);
   if (lane == 0) lmax[wave] = L;
 
-  // the query operand (head 32m + j, dims 16 s + 8 h .. + 7 at step s; zero heads past Hi) and head weights in the
-  // accumulator layout (register r of head tile m: head 32m + 8(r/4) + 4h + r%4)
+  // the query operand (head 32m + j, dims 16 s + 8 h .. + 7 at step s; zero heads past Hi)
   bf16x8 qa[MT][8];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -127,16 +141,11 @@ __global__ __launch_bounds__(PF_THREADS, MT == 1 ? 3 : 2) void indexer_prefill_k
       qa[m][s] = as_bf16x8(head < Hi ? v : make_uint4(0, 0, 0, 0));
     }
   }
-  float wr[MT][16];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int head = 32 * m + 8 * (r >> 2) + 4 * h + (r & 3);
-      const float x = w[(size_t)nq * Hi + min(head, Hi - 1)];
-      wr[m][r] = head < Hi ? x : 0.0f;
-    }
+  const float w_lane = w[(size_t)nq * Hi + min(lane, Hi - 1)];
+  wsum[wave][lane] = lane < Hi ? w_lane : 0.0f;
   __syncthreads();
+  float wr[MT][16];
+  head_weights<MT>(wsum[wave], h, wr);
   const int wg_L = max(max(lmax[0], lmax[1]), max(lmax[2], lmax[3]));
 
   float* srow = scores + (size_t)n * stride;
@@ -239,43 +248,69 @@ typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8;
 
 __device__ __forceinline__ int pf8_slot(int key, int piece) { return 8 * key + (piece ^ ((key ^ (key >> 3)) & 7)); }
 
+// Two 32-lane halves summed: lane j < 32 gets a[j] + a[j + 32], lane j + 32 gets b[j] + b[j + 32] (the key sums of two
+// tiles, one swap). v_permlane32_swap_b32 exchanges a's upper half with b's lower one; the waits that a vector write
+// before it and a read after it need are in the statement.
+__device__ __forceinline__ float half_sums(float a, float b) {
+  asm volatile("s_nop 3\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 3" : "+v"(a), "+v"(b));
+  return a + b;
+}
+
+// What bounds it: vector issue. A wave's tile (32 keys, 64 heads) is about 91 instructions, 64 of them the relu and
+// multiply-add of the products' results, which two waves a SIMD issue at one per 4.5 cycles: 824 cycles a tile and pair,
+// with the 4 products (64 cycles each) behind them. Taken out one at a time, in a copy, the head sum was worth 18%, the
+// staging 12%, the score stores 6%. So nothing else may cost an instruction or a wait: tile t's products are issued
+// between quarters of tile t - 1's head sum (two accumulator sets), its key operand is read from LDS one tile ahead, the
+// barrier of a round stands in the middle of the round before the one that it publishes (three LDS buffers, two rounds in
+// flight), the halves of the head sum are exchanged in registers, two tiles at once, scores and keys go through buffer
+// descriptors that check the bounds themselves, only tiles with a candidate are computed, and the head weights come
+// through LDS (as 32 loads a lane they were 14,000 of a workgroup's 67,000 cycles). The order of every sum is that of the
+// bf16 form above. Queries x keys, 64 heads: 2,048 x 67,584 1,225 us -> 1,178 (1.90 PF), 228 x 65,764 142 -> 137,
+// 1,001 x 7,001 72 -> 65, 256 x 16,640 49 -> 42. 3 workgroups a CU with single buffers and rounds of 2, as before, hid
+// the waits less well than this does.
 template <int MT>
-__global__ __launch_bounds__(PF_THREADS, 3) void indexer_prefill_fp8_kernel(
+__global__ __launch_bounds__(PF_THREADS, 2) void indexer_prefill_fp8_kernel(
     const uint8_t* __restrict__ q8, const float* __restrict__ qscale, const float* __restrict__ w,
     const uint8_t* __restrict__ kcache, const float* __restrict__ kscale, const int* __restrict__ npool,
     float* __restrict__ scores, int N, int Hi, int P, int stride, float scale, float* __restrict__ bm, int sub_log2,
     int nb) {
-  __shared__ u32x4 kb[2][PF8_TPB][PF_TILE * 8];  // two rounds of FP8 tiles (key j: 8 pieces of 16 bytes)
+  __shared__ u32x4 kb[3][PF8_TPB][PF_TILE * 8];  // three rounds of FP8 tiles (key j: 8 pieces of 16 bytes)
+  alignas(16) __shared__ float wsum[PF_QPW][WAVE];  // each query's head weights (times the query scales)
   __shared__ float ksc_s[PF_TILES * PF_TILE];
   __shared__ int lmax[PF_QPW];
-  const int wave = threadIdx.x / WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x & (WAVE - 1);
   const int j = lane & 31;
   const int h = lane >> 5;
   const int n = blockIdx.x * PF_QPW + wave;
-  const int nq = min(n, N - 1);
+  const int nq = min(n, N - 1);  // a wave past N computes a copy of the last query and stores nothing
   const int p_begin = blockIdx.y * PF_TILES * PF_TILE;
   const int p_end = min(p_begin + PF_TILES * PF_TILE, stride);
-  const int ntiles = (p_end - p_begin + PF_TILE - 1) / PF_TILE;
 
   const int tk = threadIdx.x >> 3, tp = threadIdx.x & 7;
-  auto load_tile = [&](int it) {
-    const int key = min(p_begin + it * PF_TILE + tk, P - 1);
-    return *reinterpret_cast<const u32x4*>(kcache + (size_t)key * PF_D + 16 * tp);
+  // the keys from the block's first on as a buffer: a load past the last key returns zeros. The tile is part of the
+  // vector offset, which the bounds check covers (it leaves the scalar offset out)
+  const auto krsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(kcache) + (size_t)min(p_begin, P - 1) * PF_D, 0,
+      (int)min((long)(P - min(p_begin, P - 1)) * PF_D, (long)PF_TILES * PF_TILE * PF_D), 0x00020000);
+  auto load_tile = [&](int it) __attribute__((always_inline)) {
+    return __builtin_bit_cast(
+        u32x4, __builtin_amdgcn_raw_buffer_load_b128(krsrc, 16 * (int)threadIdx.x + it * PF_TILE * PF_D, 0, 0));
   };
-  u32x4 ring[PF8_RING];
+  // two rounds in flight: a wait for a load also waits for the stores before it (one counter), and the compiler counts
+  // only what every way into the loop has in flight, so with one round it waits for the last round's scores
+  u32x4 ring[2 * PF8_TPB];
 #pragma unroll
-  for (int u = 0; u < PF8_RING; ++u) ring[u] = load_tile(u);
+  for (int u = 0; u < PF8_TPB; ++u) ring[u] = load_tile(u);
 #pragma unroll
   for (int i = 0; i < PF_TILES * PF_TILE / PF_THREADS; ++i) {
     const int k = i * PF_THREADS + threadIdx.x;
-    ksc_s[k] = kscale[min(p_begin + k, P - 1)];
+    ksc_s[k] = kscale[min(p_begin + k, P - 1)] * scale;
   }
-  int L = min(max(npool[nq], 0), P);
+  const int L = min(max(npool[nq], 0), P);
   if (lane == 0) lmax[wave] = L;
 
-  // A operand: head 32 m + j, dims 64 s + 32 h .. + 31 (zero heads past Hi); head weights times the query scales in
-  // the accumulator layout (register r of head tile m: head 32 m + 8 (r / 4) + 4 h + r % 4)
+  // A operand: head 32 m + j, dims 64 s + 32 h .. + 31 (zero heads past Hi)
   i32x8 qa[MT][2];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -290,82 +325,121 @@ __global__ __launch_bounds__(PF_THREADS, 3) void indexer_prefill_fp8_kernel(
       qa[m][s] = i32x8{(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
     }
   }
-  float wr[MT][16];
+  const size_t wo = (size_t)nq * Hi + min(lane, Hi - 1);
+  const float w_lane = lane < Hi ? w[wo] * qscale[wo] : 0.0f;
+  // round 0 into its buffer, rounds 1 and 2 loading
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int u = 0; u < PF8_TPB; ++u) ring[PF8_TPB + u] = load_tile(PF8_TPB + u);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int head = 32 * m + 8 * (r >> 2) + 4 * h + (r & 3);
-      const size_t o = (size_t)nq * Hi + min(head, Hi - 1);
-      wr[m][r] = head < Hi ? w[o] * qscale[o] : 0.0f;
-    }
+  for (int u = 0; u < PF8_TPB; ++u) {
+    kb[0][u][pf8_slot(tk, tp)] = ring[u];
+    ring[u] = load_tile(2 * PF8_TPB + u);
+  }
+  wsum[wave][lane] = w_lane;
   __syncthreads();
   const int wg_L = max(max(lmax[0], lmax[1]), max(lmax[2], lmax[3]));
+  float wr[MT][16];
+  head_weights<MT>(wsum[wave], h, wr);
 
+  // the block's tiles with a candidate of any of the workgroup's queries; the positions past them hold NEG_INF
   float* srow = scores + (size_t)n * stride;
-  if (p_begin >= wg_L) {
-    if (n < N) {
-      for (int p = p_begin + lane; p < p_end; p += WAVE) srow[p] = NEG_INF;
-      if (bm)
-        for (int b = (p_begin >> sub_log2) + lane; b < nb && (b << sub_log2) < p_end; b += WAVE)
-          bm[(size_t)n * nb + b] = NEG_INF;
-    }
-    return;
+  const int live = (min(p_end, wg_L) - p_begin + PF_TILE - 1) / PF_TILE;
+  const int rounds = live > 0 ? (live + PF8_TPB - 1) / PF8_TPB : 0;
+  if (n < N) {
+    for (int p = p_begin + rounds * PF8_TPB * PF_TILE + lane; p < p_end; p += WAVE) srow[p] = NEG_INF;
+    if (rounds == 0 && bm)
+      for (int b = (p_begin >> sub_log2) + lane; b < nb && (b << sub_log2) < p_end; b += WAVE)
+        bm[(size_t)n * nb + b] = NEG_INF;
   }
+  if (rounds == 0) return;
 
-  auto epilogue_part = [&](float& part, const f32x16(&prev)[MT], int s) {  // 8 of the 16 registers per step
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int e = 8 * s; e < 8 * s + 8; ++e) part = fmaf(wr[m][e], relu(prev[m][e]), part);
+  // the row's block as a buffer: a store past its end (or of a wave past N) is dropped
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(scores + (size_t)nq * stride + p_begin, 0,
+                                                      n < N ? 4 * (p_end - p_begin) : 0, 0x00020000);
+  const int slot0 = pf8_slot(j, 2 * h), slot1 = pf8_slot(j, 2 * h + 1);  // the key operand's pieces, step 0 ...
+  const int slot2 = pf8_slot(j, 4 + 2 * h), slot3 = pf8_slot(j, 5 + 2 * h);  // ... and step 1
+  u32x4 kv[2][4];
+  auto read_tile = [&](const u32x4* tile, u32x4(&o)[4]) __attribute__((always_inline)) {
+    o[0] = tile[slot0];
+    o[1] = tile[slot1];
+    o[2] = tile[slot2];
+    o[3] = tile[slot3];
   };
-  auto finish = [&](float part, int t) {
-    part += __shfl_xor(part, 32, WAVE);
-    const int pos = p_begin + t * PF_TILE + j;
-    const float v = pos < L ? part * (ksc_s[t * PF_TILE + j] * scale) : NEG_INF;
-    if (n < N && h == 0 && pos < p_end) srow[pos] = v;
-  };
-  auto tile_mma = [&](const u32x4* tile, int t, f32x16(&cur)[MT], const f32x16(&prev)[MT]) {
-    float part = 0.0f;
+  f32x16 acc[2][MT];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const u32x4 b0 = tile[pf8_slot(j, 4 * s + 2 * h)], b1 = tile[pf8_slot(j, 4 * s + 2 * h + 1)];
-      const i32x8 kbv = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3], (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
+  for (int m = 0; m < MT; ++m) acc[1][m] = f32x16{};
+  float part[2] = {0.0f, 0.0f};
+  // quarter `k` of the head sum of the tile in accumulators a, into p: at 64 heads registers 0-7 of head tiles 0 and 1,
+  // then registers 8-15 of both
+  auto head_sum = [&](float& p, const f32x16(&a)[MT], int k) __attribute__((always_inline)) {
+    constexpr int PER = 16 * MT / 4;
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        cur[m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(qa[m][s], kbv, s == 0 ? f32x16{} : cur[m], 0, 0, 0,
-                                                                 127, 0, 127);
-      epilogue_part(part, prev, s);
+    for (int i = 0; i < PER; ++i) {
+      const int m = MT == 2 ? k & 1 : 0, e = PER * (MT == 2 ? k >> 1 : k) + i;
+      p = fmaf(wr[m][e], relu(a[m][e]), p);
     }
-    if (t > 0) finish(part, t - 1);
   };
-  f32x16 acc_a[MT], acc_b[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) acc_b[m] = f32x16{};
-  auto round = [&](int t0, auto base) {
-    constexpr int U0 = decltype(base)::value;
-    u32x4(*tiles)[PF_TILE * 8] = kb[(t0 / PF8_TPB) & 1];
+  const int lim = L - p_begin;  // the query's candidates in the block
+  auto store_pair = [&](int t, float ks) __attribute__((always_inline)) {  // tiles t, t + 1: key 32 t + lane
+    const int k = t * PF_TILE + lane;
+    const float v = half_sums(part[0], part[1]) * ks;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, k < lim ? v : NEG_INF), rsrc, 4 * k, 0, 0);
+    part[0] = part[1] = 0.0f;
+  };
+  read_tile(kb[0][0], kv[0]);
+  int cur = 0;  // the round's buffer
+  auto round = [&](int r, auto base) __attribute__((always_inline)) {
+    constexpr int U0 = decltype(base)::value;  // the ring half that holds round r + 1
+    const int nxt = cur == 2 ? 0 : cur + 1;
 #pragma unroll
     for (int u = 0; u < PF8_TPB; ++u) {
-      tiles[u][pf8_slot(tk, tp)] = ring[U0 + u];
-      ring[U0 + u] = load_tile(t0 + u + PF8_RING);
-    }
-    __syncthreads();
+      const int t = r * PF8_TPB + u, c = u & 1;
+      // the next tile's key operand (after the round's last tile: the next round's first, whose buffer this round's
+      // barrier has published; past the last round it reads stale bytes that nothing uses)
+      read_tile(u + 1 < PF8_TPB ? kb[cur][u + 1] : kb[nxt][0], kv[c ^ 1]);
+      float ks = 0.0f;
+      if (c == 0) ks = ksc_s[max(t - 2, 0) * PF_TILE + lane];
+      const i32x8 b0 = {(int)kv[c][0][0], (int)kv[c][0][1], (int)kv[c][0][2], (int)kv[c][0][3],
+                        (int)kv[c][1][0], (int)kv[c][1][1], (int)kv[c][1][2], (int)kv[c][1][3]};
+      const i32x8 b1 = {(int)kv[c][2][0], (int)kv[c][2][1], (int)kv[c][2][2], (int)kv[c][2][3],
+                        (int)kv[c][3][0], (int)kv[c][3][1], (int)kv[c][3][2], (int)kv[c][3][3]};
+      // tile t's products between the quarters of tile t - 1's head sum
 #pragma unroll
-    for (int u = 0; u < PF8_TPB; u += 2) {
-      tile_mma(tiles[u], t0 + u, acc_a, acc_b);
-      tile_mma(tiles[u + 1], t0 + u + 1, acc_b, acc_a);
+      for (int i = 0; i < 4; ++i) {
+        const int s = MT == 2 ? i >> 1 : i, m = MT == 2 ? i & 1 : 0;
+        if (MT == 2 || i < 2)
+          acc[c][m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(qa[m][s], s ? b1 : b0, s ? acc[c][m] : f32x16{},
+                                                                      0, 0, 0, 127, 0, 127);
+        head_sum(part[c ^ 1], acc[c ^ 1], i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (u == 0) {  // the next round into its buffer (last read two rounds ago), the one three ahead loading
+#pragma unroll
+        for (int v = 0; v < PF8_TPB; ++v) {
+          kb[nxt][v][pf8_slot(tk, tp)] = ring[U0 + v];
+          ring[U0 + v] = load_tile((r + 3) * PF8_TPB + v);
+        }
+      }
+      if (c == 0) {
+        if (t >= 2) store_pair(t - 2, ks);
+        else part[0] = part[1] = 0.0f;
+      }
+      if (u == 1) __syncthreads();
     }
+    cur = nxt;
   };
-  int t = 0;
-  for (; t < ntiles; t += PF8_RING) {
-    round(t, std::integral_constant<int, 0>{});
-    round(t + PF8_TPB, std::integral_constant<int, PF8_TPB>{});
+  for (int r = 0;;) {
+    round(r, std::integral_constant<int, PF8_TPB>{});
+    if (++r == rounds) break;
+    round(r, std::integral_constant<int, 0>{});
+    if (++r == rounds) break;
   }
-  float part = 0.0f;
 #pragma unroll
-  for (int s = 0; s < 2; ++s) epilogue_part(part, acc_b, s);
-  finish(part, t - 1);
+  for (int i = 0; i < 4; ++i) head_sum(part[1], acc[1], i);
+  {
+    const int t = rounds * PF8_TPB - 2;
+    store_pair(t, ksc_s[t * PF_TILE + lane]);
+  }
   if (bm) {
     __syncthreads();  // the workgroup's scores are written
     if (n < N) block_max_rows(srow, 0, bm + (size_t)n * nb, p_begin, p_end, sub_log2, nb, (stride & 3) == 0, lane);
