@@ -176,6 +176,35 @@ def test_many_row_form_in_splits(B, H, keep):
     assert (lse.cpu()[~live] < -1e29).all()
 
 
+@pytest.mark.parametrize("keep, splits, form", [
+    (2048, 3, "wide"), (2048, 2, "wide"), (2048, 0, "wide"),  # all its splits, fewer, one
+    (4160, 3, "wide"), (4160, 2, "wide"), (4160, 0, "split"),  # one split is longer than its slot lists: the split form
+])
+def test_many_row_form_within_the_workspace(keep, splits, form):
+    """70 rows, 3 splits where the workspace holds them: a workspace of the split outputs of fewer (a byte short of one
+    more), or of none, is taken as the split form's own needs are (none here), and gives the same result."""
+    from tests._helpers import launched_kernels
+    B, H, L, ps = 70, 64, 4224, 64
+    g = torch.Generator().manual_seed(keep + splits)
+    say(f"attention many-row form keep={keep} in a workspace for {splits} splits")
+    kv, ks = W.quantize_rows(torch.randn(L + ps, 576, generator=g))
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    q = torch.randn(B, H, 576, generator=g).to(torch.bfloat16)
+    cnt = torch.randint(1, keep + 1, (B,), generator=g)
+    cnt[:2] = torch.tensor([keep, 1])
+    idx = torch.stack([torch.randperm(L, generator=g)[:keep] for _ in range(B)])
+    size = B * (splits + 1) * H * (512 * 4 + 8) + 256 - 1 if splits else 256
+    args = (q.cuda(), kv.cuda(), ks.cuda(), idx.cuda(), cnt.cuda(), table.cuda(), ps, 192 ** -0.5)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    names = launched_kernels(lambda: dsa_decode.attend_tokens(*args, workspace=ws))
+    kernel = "sparse_mla_wide_kernel" if form == "wide" else "sparse_mla_kernel"
+    assert names == [kernel] + ["combine_splits_kernel"] * (splits > 0), names
+    o, lse = dsa_decode.attend_tokens(*args, workspace=ws)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, 192 ** -0.5)
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-4)
+
+
 @pytest.mark.parametrize("rows_form", [False, True])
 @pytest.mark.parametrize("dqk", [576, 512])
 def test_many_row_form_moving_maxima(dqk, rows_form):

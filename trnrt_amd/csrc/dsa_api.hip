@@ -101,6 +101,7 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
                              float* lse, void* ws, int B, int H, int Dqk, int keep, int max_pages, int page_size,
                              int num_pages, float scale, int splits, hipStream_t s, PoolForm pf = PoolForm{},
                              bool wide = false);
+bool attention_wide_fits(int keep, int splits);
 int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int num_cu);
 hipError_t launch_token_rows(const int* idx, const int* cnt, const int* table, int* rows, float* bias, int B,
                              int keep, int max_pages, int page_size, int num_pages, hipStream_t s);
@@ -180,11 +181,20 @@ size_t attention_bytes(int B, int H, int keep, int tail, int splits) {
 // rows 137 and 49; 32 heads: 48 rows 145 and 92. (At 9 to 16 rows, two launches, they are 46-51 and 41-44.)
 constexpr int kBatchRows = 16;
 
-// The decode layer's attention within the workspace it is given: the many-row form in as many of its splits as fit.
-AttPlan layer_attention_plan(int B, int H, int keep, int splits, size_t bytes) {
-  AttPlan p = attention_plan(B, H, keep, 0, false, splits);
-  while (p.wide && p.splits > 1 && dsa::attention_workspace_bytes(B, H, p.splits) > bytes)
-    p.splits = effective_splits(p.splits - 1, keep);
+// The split form's workspace: the least that the attention runs in.
+size_t split_attention_bytes(int B, int H, int keep, int splits) {
+  return dsa::attention_workspace_bytes(B, H, effective_splits(resolve_splits(splits, B, H, keep), keep));
+}
+
+// The attention within the workspace that it is given (split_attention_bytes at least): the many-row form in as many of
+// its splits as fit, the split form where a split would be longer than the many-row form's slot lists.
+AttPlan fitting_plan(int B, int H, int keep, int tail, bool has_bias, int splits, size_t bytes) {
+  AttPlan p = attention_plan(B, H, keep, tail, has_bias, splits);
+  while (p.wide && dsa::attention_workspace_bytes(B, H, p.splits) > bytes) {
+    p.splits = effective_splits(p.splits - 1, keep + tail);
+    if (!dsa::attention_wide_fits(keep + tail, p.splits))
+      return {false, effective_splits(resolve_splits(splits, B, H, keep), keep)};
+  }
   return p;
 }
 
@@ -680,9 +690,9 @@ static int sparse_mla_decode(const void* q_bf16, const uint8_t* kv_fp8, const fl
   if ((Dqk != 576 && Dqk != 512) || Dv != 512 || H % 16) return DSA_EUNSUPPORTED;
   if ((long)num_pages * page_size > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (B == 0) return DSA_OK;
-  const AttPlan plan = attention_plan(B, H, keep, 0, bias != nullptr, splits);
-  const size_t need = dsa::attention_workspace_bytes(B, H, plan.splits);
+  const size_t need = split_attention_bytes(B, H, keep, splits);
   if (need && (!workspace || workspace_bytes < need)) return DSA_EWORKSPACE;
+  const AttPlan plan = fitting_plan(B, H, keep, 0, bias != nullptr, splits, workspace ? workspace_bytes : 0);
   dsa::PoolForm pf{};
   pf.n_live = n_live;
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, idx, cnt, page_table,
@@ -747,17 +757,18 @@ int dsa_sparse_mla_slots_compact(const void* q_bf16, const uint8_t* kv_fp8, cons
   if (num_slots > 0x7fffffffL || (long long)NS * kp > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (B == 0) return DSA_OK;
   const int T = NS * kp;
-  const size_t need = dsa_slots_compact_workspace_bytes(B, H, NS, kp, splits);
+  const size_t lists = align256((size_t)B * T * 4) + align256((size_t)B * 4);
+  const size_t need = lists + (H < 16 ? 0 : align256(split_attention_bytes(B, H, T, splits)));
   if (!workspace || workspace_bytes < need) return DSA_EWORKSPACE;
   auto* s = static_cast<hipStream_t>(stream);
   char* p = static_cast<char*>(workspace);
   int* tok = reinterpret_cast<int*>(p);
   int* tcnt = reinterpret_cast<int*>(p + align256((size_t)B * T * 4));
-  void* aws = p + align256((size_t)B * T * 4) + align256((size_t)B * 4);
+  void* aws = p + lists;
   if (dsa::launch_compact_slots(rows, bias, B, NS, kp, (int)(num_slots / kp), tok, tcnt, s) != hipSuccess)
     return DSA_ELAUNCH;
   // the compacted rows + count form; a row with no visible token attends its list's kp entries, all masked
-  const AttPlan plan = attention_plan(B, H, T, 0, false, splits);
+  const AttPlan plan = fitting_plan(B, H, T, 0, false, splits, workspace_bytes - lists);
   dsa::PoolForm pf{};
   pf.empty_n = kp;
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, nullptr, tcnt,
@@ -834,8 +845,9 @@ static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_
 static int pooled_layer(const void* q_idx_bf16, const float* w, const void* pool_key_bf16, const void* q_bf16,
                         const uint8_t* kv_fp8, const float* kv_scale, const int32_t* page_table, const int32_t* npool,
                         const int32_t* positions, float* scores, int32_t* pools, int32_t* cnt, void* out_bf16,
-                        float* lse, void* workspace, int B, int Hi, int H, int Dqk, int max_pages, int page_size,
-                        int num_pages, int kp, int keep, float scale, int splits, int stride, hipStream_t s);
+                        float* lse, void* workspace, size_t workspace_bytes, int B, int Hi, int H, int Dqk,
+                        int max_pages, int page_size, int num_pages, int kp, int keep, float scale, int splits,
+                        int stride, hipStream_t s);
 // The decode layer's checks, shared by its forms (every check before the first launch: a rejected call writes
 // nothing); need_ws: the caller passes a workspace (the allocation-free form checks its scratch's size itself).
 static int layer_checks(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
@@ -852,7 +864,7 @@ static int layer_checks(const void* q_idx_bf16, const float* w, const uint8_t* k
   if (Hi > 64 || page_size % 32 || H % 16) return DSA_EUNSUPPORTED;
   if ((long)num_pages * page_size > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (!dsa::topk_supported(max_len, keep, 1)) return DSA_EUNSUPPORTED;
-  if (need_ws && workspace_bytes < dsa_workspace_bytes(DSA_WS_LAYER, B, H, keep, max_len, splits))
+  if (need_ws && workspace_bytes < layer_min_bytes(B, H, keep, max_len, splits))
     return DSA_EWORKSPACE;
   return DSA_OK;
 }
@@ -986,7 +998,7 @@ static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_
   }
   char* aws = static_cast<char*>(workspace) + t_need + layer_rows_bytes(B, keep);
   const size_t aws_bytes = workspace_bytes - t_need - layer_rows_bytes(B, keep);
-  const AttPlan plan = layer_attention_plan(B, H, keep, splits, aws_bytes);
+  const AttPlan plan = fitting_plan(B, H, keep, 0, false, splits, aws_bytes);
   // the default split count on a GPU of 8 XCDs x 32 CUs, a batch of few rows (or head counts the many-row form does not
   // take): the one-launch layer's attention and combine as a launch of their own (XCD-local, bf16 split outputs),
   // over the slot rows (flat rows) or the positions through the page table
@@ -1045,9 +1057,9 @@ int dsa_sparse_mla_pooled(const void* q_bf16, const uint8_t* kv_fp8, const float
   if ((long)num_pages * page_size > 0x7fffffffL) return DSA_EUNSUPPORTED;
   if (B == 0) return DSA_OK;
   const int keep_sel = kp * keep;  // the selected pools' token slots; the tail comes on top
-  const AttPlan plan = attention_plan(B, H, keep_sel, kp, false, splits);
-  const size_t need = dsa::attention_workspace_bytes(B, H, plan.splits);
+  const size_t need = split_attention_bytes(B, H, keep_sel, splits);
   if (need && (!workspace || workspace_bytes < need)) return DSA_EWORKSPACE;
+  const AttPlan plan = fitting_plan(B, H, keep_sel, kp, false, splits, workspace ? workspace_bytes : 0);
   const dsa::PoolForm pf = {__builtin_ctz((unsigned)kp), keep, npool, positions, 0, 0, nullptr};
   return status(dsa::launch_sparse_mla(static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, pools, cnt, page_table,
                                        nullptr, nullptr, static_cast<uint16_t*>(out_bf16), out_f32, lse, workspace, B,
@@ -1055,21 +1067,27 @@ int dsa_sparse_mla_pooled(const void* q_bf16, const uint8_t* kv_fp8, const float
                                        static_cast<hipStream_t>(stream), pf, plan.wide));
 }
 
-size_t dsa_pooled_workspace_bytes(int B, int H, int keep, int max_len, int kp, int splits) {
+// The least workspace the pooled layer runs in (the many-row attention then takes the splits that fit).
+static size_t pooled_min_bytes(int B, int H, int keep, int max_len, int kp, int splits) {
   if (B < 0 || H < 16 || keep < 1 || max_len < 1 || kp < 2) return 0;
   const int keep_sel = kp * keep;
-  const int sp = effective_splits(resolve_splits(splits, B, H, keep_sel), keep_sel);
   // the split attention's workspace, or the XCD-local attention launch's (split outputs and their (max, sum))
   const size_t t = align256(dsa::topk_workspace_bytes(B, max_len, keep));
-  const size_t a = align256(dsa::attention_workspace_bytes(B, H, sp));
+  const size_t a = align256(split_attention_bytes(B, H, keep_sel, splits));
   const size_t x = align256(dsa::attend_xcd_bytes(B, H, keep_sel));
   // the one-launch form's layout shares the zero region and needs its own rest (key lists, split outputs)
   const size_t f = align256(dsa::fused_pooled_bytes(dsa::topk_zero_bytes(B), B, H));
-  const size_t w =
-      align256(dsa::attention_workspace_bytes(B, H, attention_plan(B, H, keep_sel, kp, false, splits).splits));
-  size_t chain = t + (a > x ? a : x);
-  chain = t + w > chain ? t + w : chain;
+  const size_t chain = t + (a > x ? a : x);
   return f > chain ? f : chain;
+}
+
+size_t dsa_pooled_workspace_bytes(int B, int H, int keep, int max_len, int kp, int splits) {
+  const size_t least = pooled_min_bytes(B, H, keep, max_len, kp, splits);
+  if (!least) return 0;
+  const int w = attention_plan(B, H, kp * keep, kp, false, splits).splits;
+  const size_t wide = align256(dsa::topk_workspace_bytes(B, max_len, keep)) +
+                      align256(dsa::attention_workspace_bytes(B, H, w));
+  return wide > least ? wide : least;
 }
 
 // The pooled layer's checks (every check before the first launch) and its pool stride; DSA_OK or a status.
@@ -1089,7 +1107,7 @@ static int pooled_checks(const void* q_idx_bf16, const float* w, const void* poo
   const int stride = (int)stride_l;
   if (Hi > 64 || H % 16 || (Dqk != 512 && Dqk != 576)) return DSA_EUNSUPPORTED;
   if (!dsa::topk_supported(stride, keep, 1)) return DSA_EUNSUPPORTED;
-  if (workspace_bytes < dsa_pooled_workspace_bytes(B, H, keep, stride, kp, splits)) return DSA_EWORKSPACE;
+  if (workspace_bytes < pooled_min_bytes(B, H, keep, stride, kp, splits)) return DSA_EWORKSPACE;
   *stride_out = stride;
   return DSA_OK;
 }
@@ -1180,8 +1198,8 @@ int dsa_pooled_decode_layer_chain(const void* q_idx_bf16, const float* w, const 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (ready_zero(workspace, dsa::topk_zero_bytes(B), s) != hipSuccess) return DSA_ELAUNCH;
   const int r = pooled_layer(q_idx_bf16, w, pool_key_bf16, q_bf16, kv_fp8, kv_scale, page_table, npool, positions,
-                             scores, pools, cnt, out_bf16, lse, workspace, B, Hi, H, Dqk, max_pages, page_size,
-                             num_pages, kp, keep, scale, splits, stride, s);
+                             scores, pools, cnt, out_bf16, lse, workspace, workspace_bytes, B, Hi, H, Dqk, max_pages,
+                             page_size, num_pages, kp, keep, scale, splits, stride, s);
   if (r != DSA_OK) drop_zero(workspace);
   return r;
 }
@@ -1192,8 +1210,9 @@ int dsa_pooled_decode_layer_chain(const void* q_idx_bf16, const float* w, const 
 static int pooled_layer(const void* q_idx_bf16, const float* w, const void* pool_key_bf16, const void* q_bf16,
                         const uint8_t* kv_fp8, const float* kv_scale, const int32_t* page_table, const int32_t* npool,
                         const int32_t* positions, float* scores, int32_t* pools, int32_t* cnt, void* out_bf16,
-                        float* lse, void* workspace, int B, int Hi, int H, int Dqk, int max_pages, int page_size,
-                        int num_pages, int kp, int keep, float scale, int splits, int stride, hipStream_t s) {
+                        float* lse, void* workspace, size_t workspace_bytes, int B, int Hi, int H, int Dqk,
+                        int max_pages, int page_size, int num_pages, int kp, int keep, float scale, int splits,
+                        int stride, hipStream_t s) {
   const int ppp = page_size / kp;  // pools per page
   const size_t t_need = align256(dsa::topk_workspace_bytes(B, stride, keep));
   // flat rows: the indexer accumulates the top-k's first-level histogram (the workspace's first region)
@@ -1214,7 +1233,7 @@ static int pooled_layer(const void* q_idx_bf16, const float* w, const void* pool
   // the default split count on a GPU of 8 XCDs x 32 CUs, 512-wide rows: the attention and combine in one XCD-local
   // launch (the separate kernels' form of the one-launch layer's last stages), the tail in the split of the last
   // selected token; the barrier words are the workspace's first bytes (a batch of many rows: the many-row form)
-  const AttPlan plan = attention_plan(B, H, keep_sel, kp, false, splits);
+  const AttPlan plan = fitting_plan(B, H, keep_sel, kp, false, splits, workspace_bytes - t_need);
   if (splits == 0 && dsa::attend_xcd_pooled_ok(num_cu(), H, Dqk, keep_sel) && !(plan.wide && B > kBatchRows))
     return status(dsa::launch_decode_attend_pooled(
         static_cast<const uint16_t*>(q_bf16), kv_fp8, kv_scale, pools, cnt, npool, positions, page_table,

@@ -490,6 +490,11 @@ int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int
   return sps <= AW_MAXSLOTS ? (keep + sps - 1) / sps : 0;
 }
 
+// Whether `keep` slots in this many splits fit the kernel's slot lists.
+bool attention_wide_fits(int keep, int splits) {
+  return splits > 0 && ((keep + splits - 1) / splits + AW_CH - 1) / AW_CH * AW_CH <= AW_MAXSLOTS;
+}
+
 hipError_t launch_sparse_mla_wide(const uint16_t* q, const uint8_t* kv, const float* kvs, const int* idx,
                                   const int* cnt, const int* table, const int* rows, uint16_t* out, float* out_f32,
                                   float* lse, float* ws_o, float* ws_ml, int B, int H, int Dqk, int keep,
