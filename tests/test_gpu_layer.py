@@ -205,6 +205,10 @@ def test_layer_long_tied_row_every_tile_read():
     (64, [4097, 0, 1, 2047, 2048, 2049, 4096, 31, 33, 64, 4095, 100, 3000, 8000, 8192, 500, 7, 8191], "wide"),
     # 128 heads (two workgroups a row and split): the many-row attention from 5 rows on
     (128, [6000, 0, 2500, 1, 5999], "wide"),
+    # the one-workgroup selection's last length and its edges (groups of 4,096), and the chunked pair's first
+    (128, [16384, 0, 12289, 4096, 16383], "wide"),
+    (128, [8193, 2049, 1, 8192, 8191], "wide"),
+    (128, [16385, 16384, 2047, 0, 12288], "wide"),
     # 32 heads: the XCD-local attention launch over three rows an XCD
     (32, [9000, 0, 1, 2047, 2048, 2049, 8999, 31, 33, 64, 4095, 100, 3000, 8193, 8192, 500, 7], "xcd"),
 ])

@@ -1462,8 +1462,8 @@ static hipError_t launch_topk_chunked(const float* scores, int stride, const int
                 stride, len, len_div, len_mul, keep, vis_only, nch, tb.hist, tb.meta, tb.ckey, idx, cnt, so);
 }
 
-// The flat selection of rows of at most max_len <= TOPK_FLAT_MAX scores: one workgroup per row up to 4096 scores,
-// the chunked kernels above that.
+// The flat selection of rows of at most max_len <= TOPK_FLAT_MAX scores: one workgroup per row up to 4096 scores (16384
+// with the histogram ready) or of many rows, the chunked kernels above that.
 static hipError_t launch_topk_level(const float* scores, int stride, const int* len, int len_div, int len_mul,
                                     int max_len, int keep, int vis_only, int* idx, int* cnt, const TopkBuffers& tb,
                                     bool hist_ready, const SlotOut& so, int B, hipStream_t s) {
@@ -1474,14 +1474,20 @@ static hipError_t launch_topk_level(const float* scores, int stride, const int* 
                : launch_topk_row<1, false>(scores, stride, len, len_div, len_mul, keep, vis_only, tb.hist, hist_ready,
                                            idx, cnt, so, B, s);
   if (max_len > TC_MAXCH * TC_CHUNK) return hipErrorInvalidValue;
-  // the first-level histogram ready (the fused indexer's) and rows of at most 8192 scores: one workgroup per row,
+  // the first-level histogram ready (the fused indexer's) and rows of at most 16384 scores: one workgroup per row,
   // one kernel (measured at 8 rows: 7.3 us against 4.6 + 5.8 us for the chunked pair at 8192 scores, but 20.1 us
-  // against 4.3 + 7.4 us at 32768, where one CU per row is the bound)
-  if (hist_ready && max_len <= 8 * TR_THREADS &&
-      (!so.rows || (max_len + so.page_size - 1) / so.page_size <= TR_THREADS))
+  // against 4.3 + 7.4 us at 32768, where one CU per row is the bound; whole decode steps with it and with the pair:
+  // 12 rows of 16,384 42.5 and 43.6 us, 13 rows of 2,000 to 12,345 42.3 and 44.2, 48 rows of 12,288 60.3 and 63.1)
+  const bool one = hist_ready && (!so.rows || (max_len + so.page_size - 1) / so.page_size <= TR_THREADS);
+  if (one && max_len <= 8 * TR_THREADS)
     return vec ? launch_topk_row<2, true>(scores, stride, len, len_div, len_mul, keep, vis_only, tb.hist, true, idx,
                                           cnt, so, B, s)
                : launch_topk_row<2, false>(scores, stride, len, len_div, len_mul, keep, vis_only, tb.hist, true, idx,
+                                           cnt, so, B, s);
+  if (one && max_len <= 16 * TR_THREADS)
+    return vec ? launch_topk_row<4, true>(scores, stride, len, len_div, len_mul, keep, vis_only, tb.hist, true, idx,
+                                          cnt, so, B, s)
+               : launch_topk_row<4, false>(scores, stride, len, len_div, len_mul, keep, vis_only, tb.hist, true, idx,
                                            cnt, so, B, s);
   if (B >= TOPK_MANY_ROWS && !hist_ready && !so.rows)
     return vec ? launch_topk_many_rows<true>(scores, stride, len, len_div, len_mul, max_len, keep, vis_only, tb.hist,
