@@ -14,14 +14,15 @@ def on_gpu(*ts: torch.Tensor | None) -> torch.device:
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "trnrt_amd DSA kernels run on the GPU only (libdsa_gfx950.so); got a tensor on " + str(t.device)
             )
+        d = t.device
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} and {t.device}")
+            dev = d
+        elif d != dev:
+            raise ValueError(f"tensors on different devices: {dev} and {d}")
     if dev is None:
         raise ValueError("no tensor arguments")
     return dev
@@ -40,7 +41,7 @@ def need(t: torch.Tensor, name: str, dtype: torch.dtype | tuple, shape: tuple | 
     dts = dtype if isinstance(dtype, tuple) else (dtype,)
     if t.dtype not in dts:
         raise ValueError(f"{name}: dtype {t.dtype}, expected {' or '.join(map(str, dts))}")
-    if shape is not None:
+    if shape is not None and t.shape != shape:  # (unequal also where an entry is free)
         if t.dim() != len(shape) or any(s is not None and s != d for s, d in zip(shape, t.shape)):
             raise ValueError(f"{name}: shape {tuple(t.shape)}, expected {shape}")
     if not t.is_contiguous():

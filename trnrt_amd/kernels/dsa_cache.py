@@ -55,9 +55,12 @@ def store(cache: torch.Tensor, slots: torch.Tensor, x: torch.Tensor, fp8_max: fl
     else:
         raise ValueError(f"dsa_cache.store: rows of dtype {x.dtype}, expected bfloat16 or float32")
     x = x.contiguous()
-    slots = C.need(slots.reshape(-1).to(torch.int64).contiguous(), "slots", torch.int64, (T,))
+    # a step's two stores of a few us each are bound by this function: no tensor operation that changes nothing
+    if slots.dim() != 1 or slots.dtype != torch.int64 or not slots.is_contiguous():
+        slots = slots.reshape(-1).to(torch.int64).contiguous()
+    C.need(slots, "slots", torch.int64, (T,))
     if scale is not None:
-        scale = C.need(scale.reshape(-1), "scale", torch.float32, (num_slots,))
+        scale = C.need(scale if scale.dim() == 1 else scale.reshape(-1), "scale", torch.float32, (num_slots,))
     if not 0.0 < fp8_max <= FP8_MAX:
         raise ValueError(f"dsa_cache.store: fp8_max {fp8_max} outside (0, {FP8_MAX}]")
     st = _lib.lib().dsa_cache_write(C.ptr(x), x_fp32, C.ptr(slots), C.ptr(cache), C.ptr(scale), T, W, num_slots,
