@@ -94,6 +94,28 @@ def test_scores_fp8_queries_candidates_end_early(N, Hi, P, stride, high):
     assert torch.all(buf[0] == 7.0) and torch.all(buf[-1] == 7.0)
 
 
+@pytest.mark.parametrize("N,Hi,P,stride,high,bf16_keys", [
+    (3, 64, 9001, None, 300, False), (6, 64, 9001, 9004, 2305, False), (9, 64, 2100, None, 257, False),
+    (5, 32, 6200, 6501, 2049, False), (5, 32, 6200, 6501, 2049, True), (2, 5, 33, 35, 33, True),
+    (9, 32, 4200, None, 128, True)])
+def test_scores_bf16_queries_candidates_end_early(N, Hi, P, stride, high, bf16_keys):
+    """The bf16-query form's workgroups stop at their queries' last candidate too, by 256 keys (128 at up to 32 heads)."""
+    say(f"prefill scores bf16 q N={N} Hi={Hi} P={P} stride={stride} candidates to {high} bf16 keys {bf16_keys}")
+    npool = torch.tensor([high, 0, 1, high - 1, 257, 32, 255, 127, 128][:N]).clamp(0, high)
+    qI, w, k8, ks, npool = _inputs(N, Hi, P, seed=N + P, npool=npool)
+    keys, scale = (k8.to(torch.bfloat16), None) if bf16_keys else (k8, ks)
+    buf = torch.full((N + 2, stride or P), 7.0, device="cuda")
+    LS.scores(qI.cuda(), w.cuda(), keys.cuda(), npool.cuda(), 128 ** -0.5,
+              pk_scale=None if scale is None else scale.cuda(), stride=stride, out=buf[1:-1])
+    torch.cuda.synchronize()
+    assert torch.all(buf[0] == 7.0) and torch.all(buf[-1] == 7.0)
+    got = buf[1:-1].cpu()
+    ref = O.prefill_scores_ref(qI, w, k8, torch.ones(P) if bf16_keys else ks, npool, 128 ** -0.5, stride)
+    live = ref > -1e29
+    assert row_rel_err(got, ref, live) <= TOL
+    assert torch.all(got[~live] == O.NEG_INF)
+
+
 def test_fp8_query_argument_checks():
     qI, w, k8, ks, npool = _inputs(2, 8, 64, seed=1)
     q8, qs, _ = _fp8(qI)

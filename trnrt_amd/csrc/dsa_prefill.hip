@@ -103,7 +103,6 @@ __global__ __launch_bounds__(PF_THREADS, MT == 1 ? 3 : 2) void indexer_prefill_k
   const int nq = min(n, N - 1);  // a wave past N computes a copy of the last query and stores nothing
   const int p_begin = blockIdx.y * PF_TILES * PF_TILE;
   const int p_end = min(p_begin + PF_TILES * PF_TILE, stride);
-  const int ntiles = (p_end - p_begin + PF_TILE - 1) / PF_TILE;
 
   // this thread's share of a tile: key t / 8, bytes 16 (t % 8) .. + 15 (coalesced), converted into two pieces.
   // Tiles are prefetched RING ahead into a ring of registers that is never copied (a copy of a register whose
@@ -148,16 +147,17 @@ __global__ __launch_bounds__(PF_THREADS, MT == 1 ? 3 : 2) void indexer_prefill_k
   head_weights<MT>(wsum[wave], h, wr);
   const int wg_L = max(max(lmax[0], lmax[1]), max(lmax[2], lmax[3]));
 
+  // the block's ring turns with a candidate of any of the workgroup's queries; the positions past them hold NEG_INF
   float* srow = scores + (size_t)n * stride;
-  if (p_begin >= wg_L) {  // no query of the workgroup has a candidate in the block: no MFMA
-    if (n < N) {
-      for (int p = p_begin + lane; p < p_end; p += WAVE) srow[p] = NEG_INF;
-      if (bm)
-        for (int b = (p_begin >> sub_log2) + lane; b < nb && (b << sub_log2) < p_end; b += WAVE)
-          bm[(size_t)n * nb + b] = NEG_INF;
-    }
-    return;
+  const int live = min(p_end, wg_L) - p_begin;
+  const int ntiles = live > 0 ? (live + RING * PF_TILE - 1) / (RING * PF_TILE) * RING : 0;
+  if (n < N) {
+    for (int p = p_begin + ntiles * PF_TILE + lane; p < p_end; p += WAVE) srow[p] = NEG_INF;
+    if (ntiles == 0 && bm)
+      for (int b = (p_begin >> sub_log2) + lane; b < nb && (b << sub_log2) < p_end; b += WAVE)
+        bm[(size_t)n * nb + b] = NEG_INF;
   }
+  if (ntiles == 0) return;
 
   // The relu-weighted head sum of tile t - 1 (accumulators `prev`) runs between the MFMAs of tile t (into `cur`),
   // so the VALU work of one tile overlaps the matrix work of the next.
