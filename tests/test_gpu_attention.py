@@ -248,3 +248,52 @@ def test_many_row_form_moving_maxima(dqk, rows_form):
     assert_attention_close(o, ro)
     torch.testing.assert_close(lse.cpu()[live], rl[live], atol=1e-3, rtol=1e-4)
     assert (lse.cpu()[~live] < -1e29).all()
+
+
+LEVELS = (0.0, -40.0, -89.0, -100.0, -500.0, -2000.0, 100.0, 2000.0)  # scaled scores (natural units), by head
+
+
+def _leveled(B, H, dqk, L, ps, low, seed):
+    """Queries and a cache of one L-token context whose heads' scores lie within a few units of LEVELS (heads in turn),
+    those of the positions `low` 1,000 below that for every other group of 8 heads. Dims 0 and 1 carry the two: 8 in the
+    keys (dim 1: in the low positions' alone), level x 2 in the queries, times the softmax scale 1/16 (all exact)."""
+    g = torch.Generator().manual_seed(seed)
+    kv = torch.randn(L + ps, dqk, generator=g)
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32)
+    kv[:, 0] = 8.0
+    kv[:, 1] = 0.0
+    kv[O.token_slots(table, low, ps), 1] = 8.0
+    q = torch.randn(B, H, dqk, generator=g)
+    h = torch.arange(H)
+    q[:, :, 0] = 2.0 * torch.tensor(LEVELS)[h % 8]
+    q[:, :, 1] = torch.where(h // 8 % 2 == 1, -2000.0, 0.0)
+    return q.to(torch.bfloat16), kv.to(W.FP8), torch.ones(L + ps), table.expand(B, -1).contiguous(), 1.0 / 16
+
+
+@pytest.mark.parametrize("form", ["tokens", "rows"])
+@pytest.mark.parametrize("B, keep, dqk", [(9, 2048, 576), (9, 2048, 512), (300, 256, 576), (300, 256, 512)])
+def test_many_row_form_scores_far_from_zero(B, keep, dqk, form):
+    """Softmax does not change when a head's scores are shifted, so heads whose scores all lie far below or above 0
+    (LEVELS: past -128 in base 2, where 2^-score is infinite) are as any other, and so is a row's or a split's first
+    chunk (64 slots) that lies far below the rest: 8 splits of 256 slots (9 rows) and one split (300 rows), rows of one
+    slot, one chunk, a chunk and one, a split and one, all. Bounds: the file's; for lse 5e-3, what fp32 sums of up to
+    32,000 over 36 steps round to (32,000 x 36 x 2^-24 x the scale)."""
+    say(f"attention many-row form, scores far from zero, B={B} dqk={dqk} {form}")
+    H, L, ps = 64, 2048, 64
+    low = torch.cat([torch.arange(0, 64), torch.arange(512, 576), torch.arange(1024, 1300)])
+    q, kv, ks, table, scale = _leveled(B, H, dqk, L, ps, low, seed=B + dqk)
+    cnt = torch.randint(1, keep + 1, (B,), generator=torch.Generator().manual_seed(B))
+    cnt[:7] = torch.tensor([1, 64, 65, keep, min(keep, 513), min(keep, 577), 2])
+    idx = torch.where(torch.arange(keep) < cnt.view(-1, 1), torch.arange(keep), 0)
+    if form == "rows":
+        from trnrt_amd.kernels import dsa_slots_c
+        rows = torch.stack([O.token_slots(table[b], idx[b], ps) for b in range(B)])
+        bias = torch.where(torch.arange(keep).view(1, -1) < cnt.view(-1, 1), 0.0, O.NEG_INF)
+        o, lse = dsa_slots_c.attend(q.cuda(), kv.cuda(), rows.int().cuda(), bias.cuda(), scale, lse=True,
+                                    kc_scale=ks.cuda())
+    else:
+        o, lse = dsa_decode.attend_tokens(q.cuda(), kv.cuda(), ks.cuda(), idx.cuda(), cnt.cuda(), table.cuda(), ps,
+                                          scale)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, scale)
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu(), rl, atol=5e-3, rtol=1e-4)

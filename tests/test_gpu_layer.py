@@ -237,6 +237,21 @@ def test_layer_batch_of_many_rows(H, lengths, attend):
     assert L.status()["gave_up"] == 0
 
 
+@pytest.mark.parametrize("H, B", [(64, 17), (128, 5)])
+def test_layer_batch_scores_far_from_zero(H, B):
+    """The many-row attention of a batch step with heads whose scores all lie far from 0 (as trained heads' do): a key
+    dim of 2 for every token and query values that put head h's scores around (h % 8 - 5) x 400 in natural units."""
+    say(f"layer batch, scores far from zero, H={H}")
+    lengths = ([6000, 1, 64, 65, 2047, 3000, 5999] + [100 * i for i in range(1, 11)])[:B]
+    cfg = W.Config("layer-levels", B=B, L=max(lengths), H=H, Hi=16)
+    inp = W.make_inputs(cfg, seed=H, lengths=lengths)
+    inp.kv_scale.fill_(2.0 ** -7)
+    inp.kv_cache.view(torch.uint8)[:, 0] = torch.tensor([256.0]).to(W.FP8).view(torch.uint8)
+    inp.q[:, :, 0] = ((torch.arange(H) % 8 - 5) * (200.0 / cfg.scale)).to(torch.bfloat16)
+    L = _layer(inp.to("cuda"))
+    _attention_check(inp, L)
+
+
 def _sampled_indexer_check(g, sc, nsample=4096, seed=0):
     cfg = g.cfg
     gen = torch.Generator().manual_seed(seed)

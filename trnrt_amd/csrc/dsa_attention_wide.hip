@@ -230,7 +230,8 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
         aw_barrier();
         cm = max_nonan(cm, sh.cmax[th ^ 1][32 * hh + j]);
         const float up = c == 0 || cm > AW_SLACK ? cm : 0.0f;  // how far the maximum moves
-        const float alpha = __builtin_amdgcn_exp2f(-up);
+        // chunk 0 has nothing to rescale, and its factor would be infinite where every score is at or below -128
+        const float alpha = c == 0 ? 0.0f : __builtin_amdgcn_exp2f(-up);
         m_run += up;
         l_run *= alpha;
         psum = 0.0f;
