@@ -297,3 +297,30 @@ def test_many_row_form_scores_far_from_zero(B, keep, dqk, form):
     ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, scale)
     assert_attention_close(o, ro)
     torch.testing.assert_close(lse.cpu(), rl, atol=5e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("B, keep", [(9, 2048), (300, 256)])
+def test_many_row_form_reads_no_slot_past_the_count(B, keep):
+    """Entries of the selection past a row's count name any token, also one whose cache row was never written (NaN bytes
+    and scale): they take no part in the row, in splits or not, whatever its count."""
+    say(f"attention many-row form, unwritten cache rows past the count, B={B}")
+    g = torch.Generator().manual_seed(B)
+    H, L, ps = 64, 4096, 64
+    kv, ks = W.quantize_rows(torch.randn(L + ps, 576, generator=g))
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    q = torch.randn(B, H, 576, generator=g).to(torch.bfloat16)
+    bad = O.token_slots(table[0], torch.arange(L // 2, L), ps)
+    kv.view(torch.uint8)[bad] = 0x7F
+    ks[bad] = float("nan")
+    cnt = torch.randint(1, keep + 1, (B,), generator=g)
+    cnt[:6] = torch.tensor([1, 64, 65, keep, keep - 1, 0])
+    idx = torch.stack([torch.randperm(L // 2, generator=g)[:keep].sort().values for _ in range(B)])
+    live = torch.arange(keep) < cnt.view(-1, 1).clamp(min=1)  # (a row with none attends its first entry, masked)
+    o, lse = dsa_decode.attend_tokens(q.cuda(), kv.cuda(), ks.cuda(), torch.where(live, idx, idx + L // 2).cuda(),
+                                      cnt.cuda(), table.cuda(), ps, 192 ** -0.5)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, torch.where(live, idx, idx[:, :1]), cnt, table, ps, 192 ** -0.5)
+    assert torch.isfinite(ro[cnt > 0]).all()
+    assert_attention_close(o.cpu()[cnt > 0], ro[cnt > 0])
+    torch.testing.assert_close(lse.cpu()[cnt > 0], rl[cnt > 0], atol=1e-3, rtol=1e-4)
+    v = O.dequant(kv[O.token_slots(table[0], idx[5, :1], ps)], ks[O.token_slots(table[0], idx[5, :1], ps)])[:, :512]
+    assert_attention_close(o.cpu()[5], v.expand(H, -1))

@@ -172,10 +172,11 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
 #pragma unroll
   for (int i = 0; i < AW_SPT; ++i) {
     const int k = AW_THREADS * i + tid;
-    if (k < nch * AW_CH) {
+    if (k < nch * AW_CH) {  // (past the row's slots: weight 0, and the gather takes its last slot)
+      const float ksc = k < n ? ksc_r[i] : 0.0f;
       sh.slot[k] = slot_r[i];
-      sh.ksc[k] = ksc_r[i];
-      sh.kfac[k] = masked ? 0.0f : ksc_r[i] * sl2;
+      sh.ksc[k] = ksc;
+      sh.kfac[k] = masked ? 0.0f : ksc * sl2;
     }
   }
   if (tid < 4) sh.flag[1][tid] = 0;
@@ -319,7 +320,8 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
     const int w = wave - 4, rt = tid - AW_ROLE;
     const int gr = rt >> 2, gp = 16 * (rt & 3);  // the gather: row gr of the chunk, bytes gp + 64 i .. + 15
     const int gs = gr * AW_KROW + 16 * ((rt & 3) ^ ((gr >> 1) & 3));  // and where they go in a tile
-    auto gslot = [&](int c) __attribute__((always_inline)) { return sh.slot[min(c, nch - 1) * AW_CH + gr]; };
+    // (a list entry past the row's count may name a cache row that was never written, whose NaN times weight 0 is NaN)
+    auto gslot = [&](int c) __attribute__((always_inline)) { return sh.slot[min(c * AW_CH + gr, n - 1)]; };
     u32x4 r0[PPT];
     auto gload = [&](int slot) __attribute__((always_inline)) {
       const uint8_t* src = kv + (size_t)slot * DQK + gp;
