@@ -8,6 +8,7 @@ import torch
 
 from oracle import dsa_oracle as O
 from tests._helpers import assert_attention_close, say
+from trnrt_amd import _lib
 from trnrt_amd import workloads as W
 from trnrt_amd.kernels import dsa_decode
 
@@ -324,3 +325,27 @@ def test_many_row_form_reads_no_slot_past_the_count(B, keep):
     torch.testing.assert_close(lse.cpu()[cnt > 0], rl[cnt > 0], atol=1e-3, rtol=1e-4)
     v = O.dequant(kv[O.token_slots(table[0], idx[5, :1], ps)], ks[O.token_slots(table[0], idx[5, :1], ps)])[:, :512]
     assert_attention_close(o.cpu()[5], v.expand(H, -1))
+
+
+@pytest.mark.parametrize("B, H", [(9, 64), (48, 64), (40, 128), (100, 64)])
+def test_many_row_form_reads_no_empty_split(B, H):
+    """8, 5, 3 and 2 splits of which a row's short selection fills the first ones (each count of them, 1 and a masked row
+    included), in a workspace of NaN bytes: what a split with no slot leaves there does not reach the output."""
+    say(f"attention many-row form, empty splits in a NaN workspace, B={B} H={H}")
+    g = torch.Generator().manual_seed(B)
+    keep, L, ps = 2048, 4096, 64
+    kv, ks = W.quantize_rows(torch.randn(L + ps, 576, generator=g))
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    q = torch.randn(B, H, 576, generator=g).to(torch.bfloat16)
+    cnt = torch.randint(1, 500, (B,), generator=g)
+    cnt[:9] = torch.tensor([0, 1, 256, 257, 769, 1025, 1400, 1793, 2048])
+    idx = torch.stack([torch.randperm(L, generator=g)[:keep].sort().values for _ in range(B)])
+    idx[0] = 0
+    ws = torch.full((_lib.workspace_bytes(_lib.DSA_WS_ATTENTION, B, H, keep, 0, 0),), 0xFF, dtype=torch.uint8,
+                    device="cuda")
+    o, lse = dsa_decode.attend_tokens(q.cuda(), kv.cuda(), ks.cuda(), idx.cuda(), cnt.cuda(), table.cuda(), ps,
+                                      192 ** -0.5, workspace=ws)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, 192 ** -0.5)
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu()[1:], rl[1:], atol=1e-3, rtol=1e-4)
+    assert (lse.cpu()[0] < -1e29).all()

@@ -423,26 +423,43 @@ __global__ __launch_bounds__(ATT_THREADS, 1) void sparse_mla_kernel(
 // o = sum_s W_s o_s / sum_s W_s with W_s = l_s exp(m_s - M), M = max_s m_s, and lse = M + log sum_s W_s, per
 // (sequence, head), from each split's normalised o_s, max m_s and sum l_s (the log-sum-exp combine of
 // trnrt/models/mla.py:853-856 with lse_s = m_s + log l_s kept in two parts); 128 threads x 4 dims. Every load is
-// issued before any is used (one memory round trip; unconditional, so the waits count exactly); an empty split's
-// o_s is 0 and its weight 0.
-template <int S>
+// issued before any is used (one memory round trip; unconditional, so the waits count exactly). An empty split of the
+// split form has o_s 0 and weight 0. The many-row form (MANY) leaves its empty splits' o_s unwritten, so only o_0 is read
+// before the sums are there; the others' loads follow them, a split with no slot repeating o_0's. That wait costs 0.1 to
+// 0.2 us of a step whose splits are all full (13 rows, 128 heads: 42.45 -> 42.55 us); the zeros that it saves, 128 KiB a
+// split written and read, cost 30 rows of 40 slots (keep 2,048, 8 splits, 64 heads) 22.1 us against 18.9, 16 rows of 300
+// 20.6 against 19.5, a step of 17 rows of up to 300 tokens and 128 heads 37.8 against 30.9. S is the next of 2, 4 and 8:
+// a thread's loads past the splits cost 128 rows in 2 splits 2 us.
+template <int S, bool MANY>
 __global__ __launch_bounds__(128) void combine_splits_kernel(const float* __restrict__ ws_o,
                                                              const float* __restrict__ ws_ml, int H, int splits,
                                                              uint16_t* __restrict__ out, float* __restrict__ out_f32,
                                                              float* __restrict__ lse_out,
                                                              const int* __restrict__ n_live) {
-  const int bh = blockIdx.x;
-  const int b = bh / H, head = bh - b * H;
-  if (n_live && b >= *n_live) return;  // a row past the run-time live count: left unwritten
+  // (the many-row form has at most 128 rows where it has splits: a grid of two dimensions, no division)
+  const int b = MANY ? blockIdx.y : blockIdx.x / H, head = MANY ? blockIdx.x : blockIdx.x - b * H;
+  if (!MANY && n_live && b >= *n_live) return;  // a row past the run-time live count: left unwritten
   const int d = 4 * threadIdx.x;
+  // split s of the row: its o_s at o + s so, its (m_s, l_s) at m + s sm
+  const size_t i0 = (size_t)b * splits * H + head;
+  const float* o = ws_o + i0 * ATT_DV + d;
+  const float* m = ws_ml + 2 * i0;
+  const int so = H * ATT_DV, sm = 2 * H;
   float2 ml[S];
   float4 v[S];
+  constexpr int FIRST = MANY ? 1 : S;  // split 0 always holds slots
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const size_t i = ((size_t)b * splits + min(s, splits - 1)) * H + head;
-    ml[s] = *reinterpret_cast<const float2*>(&ws_ml[2 * i]);
-    v[s] = *reinterpret_cast<const float4*>(&ws_o[i * ATT_DV + d]);
+    ml[s] = *reinterpret_cast<const float2*>(m + (size_t)min(s, splits - 1) * sm);
+    if (s < FIRST) v[s] = *reinterpret_cast<const float4*>(o + (size_t)min(s, splits - 1) * so);
   }
+  if (MANY) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int s = FIRST; s < S; ++s) {  // (as whole numbers: a scalar compare; l_s is +0 or not)
+    const size_t at = (size_t)min(s, splits - 1) * so;
+    v[s] = *reinterpret_cast<const float4*>(o + (__float_as_int(ml[s].y) ? at : 0));
+  }
+  if (MANY && n_live && b >= *n_live) return;
   float M = -INFINITY;
 #pragma unroll
   for (int s = 0; s < S; ++s) M = s < splits ? fmaxf(M, ml[s].x) : M;
@@ -533,16 +550,28 @@ size_t attention_workspace_bytes(int B, int H, int splits) {
   return (size_t)B * splits * H * ATT_DV * 4 + (size_t)B * splits * H * 8 + 256;
 }
 
-static hipError_t combine(const float* ws_o, const float* ws_ml, int B, int H, int splits, uint16_t* out,
+static hipError_t combine(const float* ws_o, const float* ws_ml, int B, int H, int splits, bool many, uint16_t* out,
                           float* out_f32, float* lse, const int* n_live, hipStream_t s) {
   const dim3 grid(B * H), block(128);
+  if (many && splits > 8) return hipErrorInvalidValue;  // (attention_wide_splits)
+  if (many) {
+    const dim3 grid2(H, B);
+    if (splits <= 2)
+      return launch("combine_splits_kernel", combine_splits_kernel<2, true>, grid2, block, s, ws_o, ws_ml, H, splits,
+                    out, out_f32, lse, n_live);
+    if (splits <= 4)
+      return launch("combine_splits_kernel", combine_splits_kernel<4, true>, grid2, block, s, ws_o, ws_ml, H, splits,
+                    out, out_f32, lse, n_live);
+    return launch("combine_splits_kernel", combine_splits_kernel<8, true>, grid2, block, s, ws_o, ws_ml, H, splits, out,
+                  out_f32, lse, n_live);
+  }
   if (splits <= 8)
-    return launch("combine_splits_kernel", combine_splits_kernel<8>, grid, block, s, ws_o, ws_ml, H, splits, out,
+    return launch("combine_splits_kernel", combine_splits_kernel<8, false>, grid, block, s, ws_o, ws_ml, H, splits, out,
                   out_f32, lse, n_live);
   if (splits <= 16)
-    return launch("combine_splits_kernel", combine_splits_kernel<16>, grid, block, s, ws_o, ws_ml, H, splits, out,
-                  out_f32, lse, n_live);
-  return launch("combine_splits_kernel", combine_splits_kernel<32>, grid, block, s, ws_o, ws_ml, H, splits, out,
+    return launch("combine_splits_kernel", combine_splits_kernel<16, false>, grid, block, s, ws_o, ws_ml, H, splits,
+                  out, out_f32, lse, n_live);
+  return launch("combine_splits_kernel", combine_splits_kernel<32, false>, grid, block, s, ws_o, ws_ml, H, splits, out,
                 out_f32, lse, n_live);
 }
 
@@ -569,7 +598,7 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
     const hipError_t e = launch_sparse_mla_wide(q, kv, kvs, idx, cnt, table, rows, eff > 1 ? nullptr : out,
                                                 eff > 1 ? nullptr : out_f32, lse, ws_o, ws_ml, B, H, Dqk, keep,
                                                 max_pages, page_size, num_pages, scale, eff, sps, pf, s);
-    return e != hipSuccess || eff == 1 ? e : combine(ws_o, ws_ml, B, H, eff, out, out_f32, lse, pf.n_live, s);
+    return e != hipSuccess || eff == 1 ? e : combine(ws_o, ws_ml, B, H, eff, true, out, out_f32, lse, pf.n_live, s);
   }
   // the split form adds the pooled tail apart from its keep slots when its rows fit their LDS (kpool 8 with 576-wide
   // rows: 7 x 576 bytes do not; the tail is then among the slots, keep + kpool of them)
@@ -597,7 +626,8 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
                    table, rows, bias, out, out_f32, lse, ws_o, ws_ml, B, H, keep, max_pages, page_size, num_pages,
                    scale, eff_splits, sps, pf);
   return e != hipSuccess || eff_splits == 1 ? e
-                                             : combine(ws_o, ws_ml, B, H, eff_splits, out, out_f32, lse, pf.n_live, s);
+                                             : combine(ws_o, ws_ml, B, H, eff_splits, false, out, out_f32, lse,
+                                                       pf.n_live, s);
 }
 
 hipError_t launch_token_rows(const int* idx, const int* cnt, const int* table, int* rows, float* bias, int B,

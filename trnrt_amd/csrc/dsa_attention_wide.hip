@@ -124,8 +124,7 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
   const int n_eff = cnt_b < 1 ? min(max(pf.empty_n, 1), keep) : (cnt_b > keep ? keep : cnt_b);
   const bool masked = cnt_b < 1;
   const int n = min(n_eff - k0, sps);
-  if (n <= 0) {  // only with splits: the combine gives it no weight
-    for (int i = tid; i < AW_HEADS * AW_DV; i += AW_THREADS) ws_o[hrow * AW_DV + i] = 0.0f;
+  if (n <= 0) {  // only with splits: the combine reads no outputs of a split whose sum is 0
     if (tid < AW_HEADS) {
       ws_ml[2 * (hrow + tid)] = -INFINITY;
       ws_ml[2 * (hrow + tid) + 1] = 0.0f;
