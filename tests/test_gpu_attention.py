@@ -154,7 +154,7 @@ def test_many_row_form_vs_oracle(dqk):
 
 @pytest.mark.parametrize("B,H,keep", [(9, 64, 2048), (43, 64, 2048), (5, 128, 4160), (70, 64, 192), (140, 128, 64)])
 def test_many_row_form_in_splits(B, H, keep):
-    """The many-row form in splits (from 9 workgroups' rows on; 8, 5, 8, 3 and 1 of them here), counts that leave the
+    """The many-row form in splits (from 9 workgroups' rows on; 8, 5, 8, 1 and 1 of them here), counts that leave the
     last splits empty (0, 1, one chunk, a chunk and one slot, all), against the oracle; slots of one 4,224-token context."""
     g = torch.Generator().manual_seed(B + keep)
     say(f"attention many-row form in splits B={B} H={H} keep={keep}")
@@ -349,3 +349,31 @@ def test_many_row_form_reads_no_empty_split(B, H):
     assert_attention_close(o, ro)
     torch.testing.assert_close(lse.cpu()[1:], rl[1:], atol=1e-3, rtol=1e-4)
     assert (lse.cpu()[0] < -1e29).all()
+
+
+@pytest.mark.parametrize("B, H, keep, form", [
+    (8, 64, 256, "split form"), (9, 64, 256, "one"), (5, 128, 256, "one"),  # more than 8 workgroups' rows
+    (9, 64, 512, "one"), (10, 64, 512, "split form"), (10, 64, 448, "one"),  # 8 chunks and more of up to 16 rows: by
+    (16, 64, 1024, "split form"), (16, 64, 1600, "splits"), (17, 64, 1024, "splits"),  # the split form's rounds
+    (17, 64, 640, "one"), (17, 64, 641, "splits"), (23, 64, 768, "splits"), (24, 64, 768, "one"), (24, 64, 769, "splits"),
+])
+def test_attention_form_by_rows_and_slots(B, H, keep, form):
+    """The form that splits 0 takes at the edges of its rule, and its result, against the oracle."""
+    from tests._helpers import launched_kernels
+    say(f"attention form B={B} H={H} keep={keep}")
+    g = torch.Generator().manual_seed(B + keep)
+    L, ps = 2048, 64
+    kv, ks = W.quantize_rows(torch.randn(L + ps, 576, generator=g))
+    table = (torch.randperm(L // ps, generator=g) + 1).to(torch.int32).expand(B, -1).contiguous()
+    q = torch.randn(B, H, 576, generator=g).to(torch.bfloat16)
+    cnt = torch.randint(1, keep + 1, (B,), generator=g)
+    cnt[:3] = torch.tensor([keep, 1, keep - 1])
+    idx = torch.stack([torch.randperm(L, generator=g)[:keep].sort().values for _ in range(B)])
+    args = (q.cuda(), kv.cuda(), ks.cuda(), idx.cuda(), cnt.cuda(), table.cuda(), ps, 192 ** -0.5)
+    names = launched_kernels(lambda: dsa_decode.attend_tokens(*args))
+    assert names == ["sparse_mla_kernel" if form == "split form" else "sparse_mla_wide_kernel"] + \
+        ["combine_splits_kernel"] * (form != "one"), names
+    o, lse = dsa_decode.attend_tokens(*args)
+    ro, rl = O.sparse_mla_ref(q, kv, ks, idx, cnt, table, ps, 192 ** -0.5)
+    assert_attention_close(o, ro)
+    torch.testing.assert_close(lse.cpu(), rl, atol=1e-3, rtol=1e-4)

@@ -102,7 +102,7 @@ hipError_t launch_sparse_mla(const uint16_t* q, const uint8_t* kv, const float* 
                              int num_pages, float scale, int splits, hipStream_t s, PoolForm pf = PoolForm{},
                              bool wide = false);
 bool attention_wide_fits(int keep, int splits);
-int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int num_cu);
+int attention_wide_splits(int B, int H, int keep, int tail, bool has_bias, int splits, int num_cu);
 hipError_t launch_token_rows(const int* idx, const int* cnt, const int* table, int* rows, float* bias, int B,
                              int keep, int max_pages, int page_size, int num_pages, hipStream_t s);
 int attention_default_splits(int B, int H, int keep, int num_cu);
@@ -162,7 +162,7 @@ struct AttPlan {
 };
 
 AttPlan attention_plan(int B, int H, int keep, int tail, bool has_bias, int splits) {
-  const int w = dsa::attention_wide_splits(B, H, keep + tail, has_bias, splits, num_cu());
+  const int w = dsa::attention_wide_splits(B, H, keep, tail, has_bias, splits, num_cu());
   if (w > 0) return {true, w};
   return {false, effective_splits(resolve_splits(splits, B, H, keep), keep)};
 }

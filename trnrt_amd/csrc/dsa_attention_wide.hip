@@ -28,6 +28,8 @@
 
 namespace dsa {
 
+int attention_default_splits(int B, int H, int keep, int num_cu);
+
 constexpr int AW_DV = 512;
 constexpr int AW_HEADS = 64;
 constexpr int AW_CH = 64;         // slots per chunk
@@ -474,22 +476,39 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
   }
 }
 
-// The splits this form takes a launch of B rows in, or 0 when it does not take it: 64-head workgroups, the token form
-// or rows + cnt (no bias array), at most AW_MAXSLOTS slots a split. An asked split count of 1 takes it when the rows
-// fill the GPU. Left to the library (splits 0), every launch of more than 8 workgroups' rows takes it, in as many
-// splits as keep one workgroup a CU, at most 8 (256 slots at keep 2,048: past that the fp32 split outputs cost what the
-// shorter splits gain). Measured against the split form (16 heads a workgroup), 2,048 slots of 576 bytes, attention
-// with its combine, 64 heads: 8 rows 21.5 us there and 21.9 here, 12 rows 37.7 and 22.8, 16 rows 27.4 and 23.0, 48
-// rows 70.8 and 32.7, 96 rows 125 and 47, 192 rows 219 and 63; 128 heads: 12 rows 51 and 25.5, 48 rows 116 and 45.
-int attention_wide_splits(int B, int H, int keep, bool has_bias, int splits, int num_cu) {
+// The splits this form takes a launch of B rows of up to keep + tail slots in (tail: a pooled row's tokens past its
+// selected pools'), or 0 when it does not take it: 64-head workgroups, the token form or rows + cnt (no bias array), at
+// most AW_MAXSLOTS slots a split. An asked split count of 1 takes it when the rows fill the GPU. Left to the library
+// (splits 0), launches of more than 8 workgroups' rows take it, measured against the split form (16 heads a workgroup)
+// with its combine, 64 heads, 576-byte rows, 9 to 255 workgroups' rows of 64 to 2,048 slots (us):
+// - up to 10 chunks of slots, one split and no combine: 9 rows of 128 slots 9.6 (split form 13.6, this form in 2 splits
+//   15.3), 64 rows of 256 13.0 (15.5; 4 splits 26.1), 20 rows of 512 17.3 (26.6; 8 splits 22.9), 32 of 640 19.9 (23.5; 5
+//   splits 22.7); of 11 and 12 chunks from 24 rows on: 64 rows of 768 23.4 (28.5; 4 splits 28.8);
+// - the split form instead for up to 16 rows of 8 to 24 chunks where its workgroups are all resident at once (a second
+//   round of them costs it 7 us): 10 rows of 512 16.1 (17.3 here), 9 of 640 16.3 (18.2), 16 of 1,024 20.9 (22.0), 10 of
+//   1,536 20.7 (21.3);
+// - otherwise as many splits as keep one workgroup a CU, at most 8 (256 slots at keep 2,048: past that the fp32 split
+//   outputs cost what the shorter splits gain; of 3 chunks at least past 16 rows, where they are more: 32 rows of 1,024
+//   24.7 in 6 splits, 26.1 in 8): 12 rows of 1,024 28.0 -> 20.3, of 2,048 slots 12 rows 37.1 -> 23.0, 16
+//   rows 26.5 -> 24.8, 48 rows 67.6 -> 32.6, 96 rows 115 -> 45, 200 rows 225 -> 58; 128 heads, 24 rows of 512-byte rows
+//   65 -> 31. (8 rows of 2,048, 21.5 and 21.9, stay with the split form.)
+int attention_wide_splits(int B, int H, int keep, int tail, bool has_bias, int splits, int num_cu) {
   if (B < 1 || H < AW_HEADS || H % AW_HEADS || has_bias || keep < 1 || splits > 1) return 0;
-  const long units = (long)B * (H / AW_HEADS);
-  if (splits == 1) return keep <= AW_MAXSLOTS && units >= num_cu ? 1 : 0;
+  const long units = (long)B * (H / AW_HEADS), slots = (long)keep + tail;
+  if (splits == 1) return slots <= AW_MAXSLOTS && units >= num_cu ? 1 : 0;
   if (units <= 8) return 0;
+  const long chunks = (slots + AW_CH - 1) / AW_CH;
+  if (units <= 16 && chunks >= 8 && chunks <= 24) {
+    const int sp = attention_default_splits(B, H, keep, num_cu);
+    const int sps = ((keep + sp - 1) / sp + AW_CH - 1) / AW_CH * AW_CH;
+    if (4 * units * ((keep + sps - 1) / sps) <= num_cu) return 0;
+  }
+  if (chunks <= 10 || (chunks <= 12 && units >= 24)) return 1;
   long s = num_cu / units;
   s = s < 1 ? 1 : s > 8 ? 8 : s;
-  const int sps = (int)((keep + s - 1) / s + AW_CH - 1) / AW_CH * AW_CH;
-  return sps <= AW_MAXSLOTS ? (keep + sps - 1) / sps : 0;
+  if (units > 16 && s > (chunks + 2) / 3) s = (chunks + 2) / 3;
+  const long sps = ((slots + s - 1) / s + AW_CH - 1) / AW_CH * AW_CH;
+  return sps <= AW_MAXSLOTS ? (int)((slots + sps - 1) / sps) : 0;
 }
 
 // Whether `keep` slots in this many splits fit the kernel's slot lists.
