@@ -427,7 +427,8 @@ int dsa_pool_keys_write(const void* rows, int rows_fp8, const float* rows_scale,
  */
 size_t dsa_workspace_bytes(int kind, int B, int H, int keep, int max_len, int splits);
 
-/* The split count dsa_sparse_mla_decode uses for splits = 0. */
+/* The split count that fills the GPU with the split form (16 heads a workgroup), the form that a split count above 1
+ * asks for: handed back as splits it is that form. splits = 0 itself may take another form and other splits. */
 int dsa_default_splits(int B, int H, int keep);
 
 /*

@@ -100,6 +100,15 @@ def test_supported_and_workspace():
     assert ws >= (8 * sp * 64 * 512 * 4 if sp > 1 else 0)
 
 
+def test_default_splits_are_the_split_forms():
+    """A caller that hands the count back gets the kernel that it counts for (16 heads a workgroup, about a workgroup a
+    CU of 256), also for batches that the library takes through the many-row form by itself."""
+    lib = _lib.lib()
+    for (B, H, keep), want in {(8, 64, 2048): 8, (48, 64, 2048): 2, (13, 128, 2048): 3, (1, 16, 2048): 32,
+                               (9, 64, 2048): 8, (300, 64, 2048): 1, (30, 64, 512): 3, (4, 64, 100): 2}.items():
+        assert lib.dsa_default_splits(B, H, keep) == want, (B, H, keep)
+
+
 def test_check_maps_status_to_the_reference_exceptions():
     with pytest.raises(ValueError):
         _lib.check(-1, "x")

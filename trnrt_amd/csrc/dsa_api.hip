@@ -832,7 +832,7 @@ size_t dsa_workspace_bytes(int kind, int B, int H, int keep, int max_len, int sp
 
 int dsa_default_splits(int B, int H, int keep) {
   if (B < 1 || H < 16 || keep < 1) return 1;
-  return attention_plan(B, H, keep, 0, false, 0).splits;
+  return effective_splits(resolve_splits(0, B, H, keep), keep);
 }
 
 static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,
