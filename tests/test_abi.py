@@ -100,6 +100,33 @@ def test_supported_and_workspace():
     assert ws >= (8 * sp * 64 * 512 * 4 if sp > 1 else 0)
 
 
+def _split_form_bytes(B, H, splits):
+    return B * splits * H * (512 * 4 + 8) + 256 if splits > 1 else 0
+
+
+@pytest.mark.parametrize("H", [16, 32, 64, 128, 192, 256])
+def test_size_queries_cover_the_split_form(H):
+    """Every attention call needs at least the split form's workspace (dsa_default_splits of its 16-head splits over the
+    selected tokens), whichever form runs: the queries for splits 0 return no less, over batches, head counts, selections
+    and pool sizes. A query of an explicit split count is that count's."""
+    lib = _lib.lib()
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    for B in [*range(1, 75), 100, 129, 200, 256, 257, 300]:
+        for keep in (1, 64, 80, 256, 320, 512, 1024):
+            for kp in (2, 4, 8):
+                sp = lib.dsa_default_splits(B, H, keep * kp)
+                need = _split_form_bytes(B, H, sp)
+                shape = (B, H, keep, kp)
+                assert lib.dsa_sparse_mla_pooled_workspace_bytes(*shape, 0) >= need, shape
+                assert lib.dsa_sparse_mla_pooled_workspace_bytes(*shape, sp) in (need, up(need)), shape
+                lists = up(B * keep * kp * 4) + up(B * 4)
+                assert lib.dsa_slots_compact_workspace_bytes(*shape, 0) >= lists + need, shape
+                assert lib.dsa_slots_compact_workspace_bytes(*shape, sp) == lists + up(need), shape
+                assert lib.dsa_pooled_workspace_bytes(B, H, keep, 4096, kp, 0) >= need, shape
+                assert _lib.workspace_bytes(_lib.DSA_WS_ATTENTION, B, H, keep * kp, 0, 0) >= need, shape
+                assert _lib.workspace_bytes(_lib.DSA_WS_ATTENTION, B, H, keep * kp, 0, sp) == up(need), shape
+
+
 def test_default_splits_are_the_split_forms():
     """A caller that hands the count back gets the kernel that it counts for (16 heads a workgroup, about a workgroup a
     CU of 256), also for batches that the library takes through the many-row form by itself."""

@@ -95,6 +95,48 @@ def test_attend_pooled_tails_vs_oracle(kp, dqk, splits):
     assert torch.allclose(lse.cpu(), want_lse, atol=1e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("B,H,kp,keep,dqk,form", [
+    (9, 64, 4, 512, 512, "splits"), (17, 64, 4, 512, 512, "splits"), (70, 64, 4, 512, 576, "splits"),
+    (3, 192, 4, 512, 512, "splits"), (9, 64, 8, 64, 512, "one"), (9, 64, 2, 320, 576, "split form"),
+])
+def test_attend_pooled_many_row_form_in_its_workspace(B, H, kp, keep, dqk, form):
+    """attend_pooled with 9 workgroups' rows and more (the many-row form in splits or one, or the split form), in a
+    workspace of exactly dsa_sparse_mla_pooled_workspace_bytes: every tail length, a row with no complete pool, fewer selected pools than
+    keep. The cache rows that no row attends are NaN (bytes and scale), the tokens of the tail's pool past the position
+    among them: a context's last pages hold such rows until they are written."""
+    from trnrt_amd import _lib
+    say(f"attend_pooled many-row form B={B} H={H} kp={kp} keep={keep} dqk={dqk}")
+    g = torch.Generator().manual_seed(1000 * B + kp)
+    L, ps = 4096, 64
+    npg = L // ps
+    num_pages = 1 + B * npg
+    kv, ks = W.quantize_rows(torch.randn(num_pages * ps, dqk, generator=g))
+    table = (torch.randperm(num_pages - 1, generator=g)[: B * npg] + 1).view(B, npg).to(torch.int32)
+    q = torch.randn(B, H, dqk, generator=g).to(torch.bfloat16)
+    positions = torch.randint(0, L, (B,), generator=g)
+    positions[:3] = torch.tensor([L - 2, kp - 2, kp * (keep // 2) + 1])
+    positions[3:3 + kp] = (torch.arange(kp) + 2048)[:max(0, B - 3)]
+    pools, cnt, npool = _selection(B, L, kp, keep, positions, seed=kp + B)
+    want_r, want_b = O.pool_slots_ref(pools, cnt, npool, positions, table, ps, kp, keep + 1)
+    tok = (want_r.unsqueeze(-1) * kp + torch.arange(kp)).reshape(B, -1)
+    want_o, want_lse = O.sparse_mla_slots_ref(q, kv, ks, tok, want_b.reshape(B, -1), 192 ** -0.5)
+    used = torch.zeros(num_pages * ps, dtype=torch.bool)
+    used[tok[want_b.reshape(B, -1) == 0]] = True
+    kv.view(torch.uint8)[~used] = 0x7F
+    ks[~used] = float("nan")
+    ws = torch.empty(int(_lib.lib().dsa_sparse_mla_pooled_workspace_bytes(B, H, keep, kp, 0)), dtype=torch.uint8,
+                     device="cuda")
+    args = (q.cuda(), kv.cuda(), ks.cuda(), pools.cuda(), cnt.cuda(), npool.cuda(), positions.cuda(), table.cuda(), ps,
+            kp, 192 ** -0.5)
+    from tests._helpers import launched_kernels
+    names = launched_kernels(lambda: dsa_long.attend_pooled(*args, workspace=ws))
+    assert names == ["sparse_mla_kernel" if form == "split form" else "sparse_mla_wide_kernel"] + \
+        ["combine_splits_kernel"] * (form != "one"), names
+    o, lse = dsa_long.attend_pooled(*args, lse=True, workspace=ws)
+    assert_attention_close(o, want_o)
+    torch.testing.assert_close(lse.cpu(), want_lse, atol=1e-3, rtol=1e-4)
+
+
 def _pool_setup(seed, fp8_rows, B=3, L=1024, ps=64, kp=4):
     """A GLM-like pooled cache: per token an indexer row [key 128 | gate logits 128] (bf16, or e4m3 with per-token
     scales), B sequences of L tokens through random page tables, and an empty pool-key cache."""

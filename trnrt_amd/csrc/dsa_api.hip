@@ -167,13 +167,6 @@ AttPlan attention_plan(int B, int H, int keep, int tail, bool has_bias, int spli
   return {false, effective_splits(resolve_splits(splits, B, H, keep), keep)};
 }
 
-// The larger of the workspaces of the two forms that a call may take (with a bias array or without).
-size_t attention_bytes(int B, int H, int keep, int tail, int splits) {
-  const AttPlan p = attention_plan(B, H, keep, tail, false, splits), q = attention_plan(B, H, keep, tail, true, splits);
-  const size_t a = dsa::attention_workspace_bytes(B, H, p.splits), b = dsa::attention_workspace_bytes(B, H, q.splits);
-  return a > b ? a : b;
-}
-
 // A decode batch of more rows than this takes the separate kernels even where the one-launch layer takes its shape: the
 // one launch handles 8 rows at a time, each a chain of latencies (about 25 us), where the separate kernels' grids share
 // the whole batch. Measured, 64 heads, rows of 500 to 32,768 tokens, one launch per 8 rows against the separate kernels:
@@ -184,6 +177,14 @@ constexpr int kBatchRows = 16;
 // The split form's workspace: the least that the attention runs in.
 size_t split_attention_bytes(int B, int H, int keep, int splits) {
   return dsa::attention_workspace_bytes(B, H, effective_splits(resolve_splits(splits, B, H, keep), keep));
+}
+
+// What the size queries give: the chosen form's workspace, and no less than the split form's, which every call must have
+// (a call with a bias array takes that form; the many-row form over a pooled tail may have fewer splits).
+size_t attention_bytes(int B, int H, int keep, int tail, int splits) {
+  const size_t w = dsa::attention_workspace_bytes(B, H, attention_plan(B, H, keep, tail, false, splits).splits);
+  const size_t least = split_attention_bytes(B, H, keep, splits);
+  return w > least ? w : least;
 }
 
 // The attention within the workspace that it is given (split_attention_bytes at least): the many-row form in as many of
@@ -744,7 +745,7 @@ size_t dsa_slots_compact_workspace_bytes(int B, int H, int NS, int kp, int split
   if (B < 0 || H < 16 || NS < 1 || kp < 1) return 0;
   const int T = NS * kp;
   return align256((size_t)B * T * 4) + align256((size_t)B * 4) +
-         align256(dsa::attention_workspace_bytes(B, H, attention_plan(B, H, T, 0, false, splits).splits));
+         align256(attention_bytes(B, H, T, 0, splits));
 }
 
 int dsa_sparse_mla_slots_compact(const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale,
@@ -820,14 +821,10 @@ size_t dsa_workspace_bytes(int kind, int B, int H, int keep, int max_len, int sp
   if (kind == DSA_WS_TOPK) return align256(dsa::topk_workspace_bytes(B, max_len, keep));
   if (kind == DSA_WS_ATTENTION) return H < 16 ? 0 : align256(attention_bytes(B, H, keep, 0, splits));
   if (kind != DSA_WS_LAYER) return 0;
-  size_t total = layer_min_bytes(B, H, keep, max_len, splits);
-  const AttPlan p = H < 16 ? AttPlan{false, 1} : attention_plan(B, H, keep, 0, false, splits);
-  if (p.wide) {
-    const size_t w = align256(dsa::topk_workspace_bytes(B, max_len, keep)) + layer_rows_bytes(B, keep) +
-                     align256(dsa::attention_workspace_bytes(B, H, p.splits));
-    total = w > total ? w : total;
-  }
-  return total;
+  const size_t total = layer_min_bytes(B, H, keep, max_len, splits);
+  const size_t w = align256(dsa::topk_workspace_bytes(B, max_len, keep)) + layer_rows_bytes(B, keep) +
+                   align256(H < 16 ? 0 : attention_bytes(B, H, keep, 0, splits));
+  return w > total ? w : total;
 }
 
 int dsa_default_splits(int B, int H, int keep) {
@@ -1040,8 +1037,7 @@ int dsa_decode_layer_noalloc(const void* q_idx_bf16, const float* w, const uint8
 size_t dsa_sparse_mla_pooled_workspace_bytes(int B, int H, int keep, int kp, int splits) {
   if (B < 0 || H < 16 || keep < 1 || kp < 2) return 0;
   const int keep_sel = kp * keep;  // the selected pools' token slots; the tail comes on top
-  return align256(
-      dsa::attention_workspace_bytes(B, H, attention_plan(B, H, keep_sel, kp, false, splits).splits));
+  return align256(attention_bytes(B, H, keep_sel, kp, splits));
 }
 
 int dsa_sparse_mla_pooled(const void* q_bf16, const uint8_t* kv_fp8, const float* kv_scale, const int32_t* pools,
@@ -1084,10 +1080,9 @@ static size_t pooled_min_bytes(int B, int H, int keep, int max_len, int kp, int 
 size_t dsa_pooled_workspace_bytes(int B, int H, int keep, int max_len, int kp, int splits) {
   const size_t least = pooled_min_bytes(B, H, keep, max_len, kp, splits);
   if (!least) return 0;
-  const int w = attention_plan(B, H, kp * keep, kp, false, splits).splits;
-  const size_t wide = align256(dsa::topk_workspace_bytes(B, max_len, keep)) +
-                      align256(dsa::attention_workspace_bytes(B, H, w));
-  return wide > least ? wide : least;
+  const size_t w = align256(dsa::topk_workspace_bytes(B, max_len, keep)) +
+                   align256(attention_bytes(B, H, kp * keep, kp, splits));
+  return w > least ? w : least;
 }
 
 // The pooled layer's checks (every check before the first launch) and its pool stride; DSA_OK or a status.
