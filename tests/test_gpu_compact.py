@@ -97,3 +97,24 @@ def test_value_order_with_ties(keep):
         assert torch.equal(vv[n, :c].view(torch.int32), vals[n, order].view(torch.int32))
         assert torch.all(vp[n, c:] == 0) and torch.all(vv[n, c:] == O.NEG_INF)
     assert torch.equal(vc.cpu(), cnt)
+
+
+@pytest.mark.parametrize("B", [32, 48])
+def test_slots_compact_attend_in_less_than_the_query(B):
+    """A workspace that the queried size for these rows exceeds, but not what the attention runs in (the lists and the
+    split form's 2 splits; the query's are 8 and 5 of the many-row form), is taken as dsa_decode's is; 256 bytes less
+    are not."""
+    from trnrt_amd import _lib
+    say(f"slots_c attend B={B} in a small workspace")
+    H, NS, kp, scale = 64, 512, 4, 0.0417
+    q, kv, ks, rows, bias = _slot_inputs(B, H, NS, kp, seed=B)
+    size = lambda splits: _lib.lib().dsa_slots_compact_workspace_bytes(B, H, NS, kp, splits)  # noqa: E731
+    least = size(_lib.lib().dsa_default_splits(B, H, NS * kp))
+    assert least < size(0)
+    args = (q.cuda(), kv.cuda(), rows.cuda(), bias.cuda(), scale)
+    o = dsa_slots_c.attend(*args, kc_scale=ks.cuda(), workspace=torch.empty(least, dtype=torch.uint8, device="cuda"))
+    ro, _ = O.slots_compact_ref(q.float(), kv, ks, rows, bias, scale)
+    assert_attention_close(o.cpu(), ro)
+    with pytest.raises(ValueError):
+        dsa_slots_c.attend(*args, kc_scale=ks.cuda(),
+                           workspace=torch.empty(least - 256, dtype=torch.uint8, device="cuda"))

@@ -37,7 +37,8 @@ def attend(q_lat: torch.Tensor, kc: torch.Tensor, rows: torch.Tensor, bias: torc
     [N, NS] (pool rows of the FP8 cache kc viewed as [slots / kp, kp rows]; kc [slots, 1, D] or [slots, D] e4m3fn
     with kc_scale [slots] fp32 its per-token scales, or None for the reference's unscaled cache) with bias
     [N, NS, kp] or [N, NS] fp32 (0 / NEG_INF). workspace: dsa_slots_compact_workspace_bytes(N, H, NS, kp, splits)
-    bytes (no zero fill needed), or None for one kept per stream."""
+    bytes (no zero fill needed; with less the attention takes fewer splits, down to the split form's need), or None for
+    one kept per stream."""
     dev = C.on_gpu(q_lat, kc, rows, bias, kc_scale, workspace)
     if q_lat.dim() != 3 or q_lat.shape[2] not in DQK_WIDTHS:
         raise ValueError(f"dsa_slots_c: q_lat {tuple(q_lat.shape)}, expected [N, H, 576 or 512]")
@@ -63,10 +64,8 @@ def attend(q_lat: torch.Tensor, kc: torch.Tensor, rows: torch.Tensor, bias: torc
     ls = torch.empty(N, H, dtype=torch.float32, device=dev) if lse else None
     wsb = _lib.lib().dsa_slots_compact_workspace_bytes(N, H, NS, kp, int(splits))
     ws = workspace if workspace is not None else C.cached_workspace(dev, wsb, "slots_compact")
-    if ws.numel() * ws.element_size() < wsb:
-        raise ValueError(f"dsa_slots_c.attend: workspace of {ws.numel() * ws.element_size()} bytes, needs {wsb}")
     st = _lib.lib().dsa_sparse_mla_slots_compact(
-        C.ptr(q), C.ptr(kv), C.ptr(ks), C.ptr(r), C.ptr(b), None, C.ptr(out), C.ptr(ls), C.ptr(ws), wsb, N, H, dqk,
-        NS, kp, num_slots, float(scale), int(splits), C.stream_ptr(dev))
+        C.ptr(q), C.ptr(kv), C.ptr(ks), C.ptr(r), C.ptr(b), None, C.ptr(out), C.ptr(ls), C.ptr(ws),
+        ws.numel() * ws.element_size(), N, H, dqk, NS, kp, num_slots, float(scale), int(splits), C.stream_ptr(dev))
     _lib.check(st, "dsa_slots_c.attend")
     return (out, ls) if lse else out
