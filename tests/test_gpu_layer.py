@@ -237,6 +237,29 @@ def test_layer_batch_of_many_rows(H, lengths, attend):
     assert L.status()["gave_up"] == 0
 
 
+@pytest.mark.parametrize("Hi, L, even", [(33, 8192, False), (33, 8193, True), (32, 16384, False), (32, 16385, True)])
+def test_layer_batch_indexer_split(Hi, L, even):
+    """The indexer of a batch of 17 ragged rows at the lengths where it changes from a workgroup per 512 positions to the
+    even split (later at 32 indexer heads and fewer), against the oracle, and the selection that its histogram feeds."""
+    from tests._helpers import launched_kernels
+    say(f"layer batch indexer split Hi={Hi} L={L}")
+    lengths = [L, 0, 1, 31, 33, 512, 513, 2048, 2049, L - 1, L // 2, 4095, 4097, 8000, 100, 7, 3000]
+    cfg = W.Config("layer-even", B=len(lengths), L=L, H=16, Hi=Hi)
+    inp = W.make_inputs(cfg, seed=Hi + L, lengths=lengths)
+    g = inp.to("cuda")
+    layer = _layer(g)
+    names = launched_kernels(lambda: layer.step(g.q_idx, g.w_k, g.k_cache, g.k_scale, g.q, g.kv_cache, g.kv_scale,
+                                                g.table, g.ctx_len))
+    assert names[0] == ("indexer_decode_long_kernel" if even else "indexer_decode_kernel"), names
+    torch.cuda.synchronize()
+    sc = layer.scores.cpu()
+    ref = O.indexer_ref(inp.q_idx, inp.w_k, inp.k_cache, inp.k_scale, inp.table, inp.ctx_len, 64, sc.shape[1])
+    assert row_rel_err(sc, ref, ref > -1e29) <= 1e-2
+    assert torch.all(sc[ref <= -1e29] < -1e29)
+    ri, rc = O.topk_ref(sc, cfg.keep, inp.ctx_len)
+    assert torch.equal(layer.idx.cpu().long(), ri) and torch.equal(layer.cnt.cpu().long(), rc)
+
+
 @pytest.mark.parametrize("H, B", [(64, 17), (128, 5)])
 def test_layer_batch_scores_far_from_zero(H, B):
     """The many-row attention of a batch step with heads whose scores all lie far from 0 (as trained heads' do): a key

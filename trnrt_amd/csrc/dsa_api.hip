@@ -951,9 +951,11 @@ static int layer_chain(const void* q_idx_bf16, const float* w, const uint8_t* k_
   float* tmax = la && dsa::long_attend_tiles(max_len) ? dsa::long_attend_tmax(lws, B, H, keep, max_len) : nullptr;
   hipError_t e;
   // flat rows of a batch: the long rows' indexer too, whose workgroups share the batch's live tiles evenly whatever the
-  // rows' lengths (48 rows of 500 to 32,768 tokens 97 us a step with it, 114 with a workgroup per 512 positions of the
-  // longest row's; 48 rows of 4,096: 51 and 49)
-  const bool even = !flat || (B > kBatchRows && max_len > 8192);
+  // rows' lengths, where that outweighs its own start (every workgroup reads all the lengths). A step's us with it and
+  // with a workgroup per 512 positions of the longest row's, 64 indexer heads: 48 rows of 500 to 32,768 tokens 72 and 89,
+  // of 32,768 96 and 107, 17 rows of 9,000 to 16,384 45.0 and 46.9, 48 of 4,096 level; 16 or 32 heads: 24 rows of 500 to
+  // 32,768 52.9 and 55.4, 48 of 32,768 122 and 117, 24 of 16,384 49.3 and 46.3, 24 of 9,000 45.3 and 42.4.
+  const bool even = !flat || (B > kBatchRows && max_len > (Hi > 32 ? 8192 : 16384));
   if (!even)
     e = dsa::launch_indexer_decode(static_cast<const uint16_t*>(q_idx_bf16), w, k_fp8, k_scale, page_table, ctx_len,
                                    nullptr, scores, hist, B, Hi, max_pages, page_size, num_pages, score_stride,
