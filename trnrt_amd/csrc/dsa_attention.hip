@@ -467,7 +467,7 @@ __global__ __launch_bounds__(128) void combine_splits_kernel(const float* __rest
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const float wt = (s < splits && ml[s].y > 0.0f) ? ml[s].y * __expf(ml[s].x - M) : 0.0f;
+    const float wt = (s < splits && ml[s].y > 0.0f) ? ml[s].y * (MANY ? __builtin_amdgcn_exp2f(ml[s].x - M) : __expf(ml[s].x - M)) : 0.0f;
     W += wt;
     acc.x += wt * v[s].x;
     acc.y += wt * v[s].y;
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(128) void combine_splits_kernel(const float* __rest
   }
   if (out_f32)
     *reinterpret_cast<float4*>(&out_f32[oi]) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
-  if (lse_out && threadIdx.x == 0) lse_out[(size_t)b * H + head] = M + __logf(W);
+  if (lse_out && threadIdx.x == 0) lse_out[(size_t)b * H + head] = MANY ? lse_base2(M, W) : M + __logf(W);
 }
 
 // Token positions -> cache slots and biases (the kp = 1 form of trnrt/models/dsa_long.py:189-215).

@@ -42,7 +42,7 @@ constexpr int AW_OROW = AW_DV + 8;       // staged output row (elements)
 constexpr int AW_PROW = AW_CH + 8;       // P row stride (bf16)
 constexpr float AW_SLACK = 11.5f;        // lazy rescaling (base 2): p = 2^(s - m) <= 2^11.5 between moves of m
 constexpr float AW_LOG2E = 1.44269504088896341f;
-constexpr float AW_LN2 = 0.69314718055994531f;
+constexpr float AW_LOG2E_LO = (float)(1.44269504088896341 - (double)AW_LOG2E);
 constexpr int AW_KAHEAD = 3;  // score steps whose key reads are in flight
 constexpr int AW_VAHEAD = 3;  // value steps whose operand reads are in flight
 constexpr int AW_STORE = 5;   // the value step that begins storing the next chunk's rows
@@ -134,7 +134,8 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
     return;
   }
   const int nch = (n + AW_CH - 1) / AW_CH;
-  const float sl2 = scale * AW_LOG2E;
+  // scale x log2 e to twice fp32's digits: rounded, its error would be the same for every score, and so the lse's
+  const float sl2 = scale * AW_LOG2E, sl2_lo = fmaf(scale, AW_LOG2E, -sl2) + scale * AW_LOG2E_LO;
   // slot list entries -> cache slots, the table's loads again in one round
   if (token_form) {
     int pr[AW_SPT], pg[AW_SPT];
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
       const float ksc = k < n ? ksc_r[i] : 0.0f;
       sh.slot[k] = slot_r[i];
       sh.ksc[k] = ksc;
-      sh.kfac[k] = masked ? 0.0f : ksc * sl2;
+      sh.kfac[k] = masked ? 0.0f : fmaf(ksc, sl2, ksc * sl2_lo);
     }
   }
   if (tid < 4) sh.flag[1][tid] = 0;
@@ -456,12 +457,12 @@ __global__ __launch_bounds__(AW_THREADS, 1) void sparse_mla_wide_kernel(
   }
   if (tid < AW_HEADS) {
     const float l = sh.lsum[0][tid] + sh.lsum[1][tid];
-    const float m = masked ? NEG_INF : sh.mfin[tid] * AW_LN2;
-    if (ws_o) {
+    const float m = masked ? NEG_INF : sh.mfin[tid];
+    if (ws_o) {  // base 2, as the combine of this form takes it
       ws_ml[2 * (hrow + tid)] = m;
       ws_ml[2 * (hrow + tid) + 1] = l;
     } else if (lse_out) {
-      lse_out[hrow + tid] = m + __logf(l);
+      lse_out[hrow + tid] = lse_base2(m, l);
     }
   }
   if (out) {

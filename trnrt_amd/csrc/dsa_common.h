@@ -67,6 +67,12 @@ struct PoolForm {
   int empty_n;         // rows + cnt form: the masked slots a row with cnt 0 attends (0: one)
   const int* n_live;   // null, or one int on the device: rows at or past it are neither computed nor written
 };
+// The log-sum-exp of a row from its maximum in base 2 (NEG_INF: a row with no live slot) and its sum, the product with
+// ln 2 unrounded.
+__device__ __forceinline__ float lse_base2(float m, float l) {
+  return m > NEG_INF ? fmaf(m, 0.69314718055994531f, __logf(l)) : NEG_INF + __logf(l);
+}
+
 // The pooled decode step's pool-key write, folded into the pooled layer's launch (dsa_pooled_decode_step): the
 // indexer rows cache [slots][rows_width] (e4m3 with a per-slot fp32 scale, or bf16: rows_fp8 0), the pool-position
 // bias [kpool][128] fp32 and each row's written token's cache slot.
