@@ -44,7 +44,7 @@ extern "C" {
 #define DSA_OK 0
 #define DSA_EINVAL (-1)      /* a null pointer or a size out of range */
 #define DSA_EUNSUPPORTED (-2) /* a shape these kernels do not implement */
-#define DSA_EWORKSPACE (-3)  /* workspace smaller than dsa_workspace_bytes() */
+#define DSA_EWORKSPACE (-3)  /* workspace smaller than the call can run in (the size queries give no less) */
 #define DSA_ELAUNCH (-4)     /* the HIP runtime refused a launch */
 #define DSA_ESCRATCH (-5)    /* more scratch than dsa_decode_layer_noalloc holds */
 
@@ -293,9 +293,9 @@ int dsa_decode_layer_chain(const void* q_idx_bf16, const float* w, const uint8_t
  * the process ends; its zero region kept as any workspace's: the first call on a device fills the zero region of
  * its batch size, and a call whose zero region (the barrier words and its rows' histograms) reaches past the
  * previous call's gets the difference filled on `stream` first, so calls of any batch sizes follow each other). A
- * call whose
- * dsa_workspace_bytes(DSA_WS_LAYER, B, H, keep, max_len, splits) exceeds that size returns DSA_ESCRATCH before any
- * HIP call. Every call on a GPU shares that GPU's scratch: calls that overlap on one GPU (several streams, host
+ * call that cannot run in that size returns DSA_ESCRATCH before any HIP call. dsa_workspace_bytes(DSA_WS_LAYER, B, H,
+ * keep, max_len, splits) of at most that size always runs; a batch whose query is larger may too, with fewer attention
+ * splits than in a workspace of the queried size. Every call on a GPU shares that GPU's scratch: calls that overlap on one GPU (several streams, host
  * threads) race and must be serialised by the caller. Arguments and results as dsa_decode_layer.
  */
 #define DSA_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)

@@ -168,10 +168,17 @@ AttPlan attention_plan(int B, int H, int keep, int tail, bool has_bias, int spli
 }
 
 // A decode batch of more rows than this takes the separate kernels even where the one-launch layer takes its shape: the
-// one launch handles 8 rows at a time, each a chain of latencies (about 25 us), where the separate kernels' grids share
-// the whole batch. Measured, 64 heads, rows of 500 to 32,768 tokens, one launch per 8 rows against the separate kernels:
-// 17 rows 73 and 45 us, 24 rows 75 and 52, 48 rows 151 and 71, 64 rows 215 and 85; rows of 4,096: 24 rows 69 and 39, 48
-// rows 137 and 49; 32 heads: 48 rows 145 and 92. (At 9 to 16 rows, two launches, they are 46-51 and 41-44.)
+// one launch handles 8 rows at a time, each a chain of latencies (18 to 26 us), where the separate kernels' grids share
+// the whole batch. A step's us, one launch per 8 rows and the separate kernels, 64 heads: 17 rows of up to 500 tokens 55
+// and 31, of 32,768 76 and 53, 48 rows of up to 4,096 129 and 46; 16 heads: 17 rows of up to 1,000 50 and 31, 48 rows of
+// 500 to 32,768 133 and 87; pooled: 17 rows of 32,768 63 and 42, 32 heads, 30 rows of up to 8,000 77 and 46. At 9 to 16
+// rows, two launches, the separate kernels are the faster too (9 rows of 4,096 43.0 and 32.8, 16 rows of up to 1,000 37.8
+// and 27.2, 16 of 32,768 52.0 and 51.5; pooled, 12 rows of 32,768 41.5 and 35.9): the crossover is at 8 rows, and the
+// line stands at 16 only because batches of two launches have not been moved over it.
+// The same line in the separate kernels: past it the many-row attention (17 rows of 500 to 32,768 tokens 48.7 us a step,
+// 54.9 with the XCD-local launch; 48 rows 72 and 98; pooled 17 rows of 32,768 42.1 and 46.7), up to it the XCD-local
+// launch (16 rows of 4,096 35.0, 36.5 with the many-row form; pooled 12 rows of up to 2,000 26.5 and 30.0); and the even
+// indexer (layer_chain).
 constexpr int kBatchRows = 16;
 
 // The split form's workspace: the least that the attention runs in.

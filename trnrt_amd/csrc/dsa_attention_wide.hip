@@ -1,6 +1,6 @@
-// Sparse MLA attention over many query rows for gfx950 (the arithmetic of dsa_attention.hip, for a prefill chunk's
-// queries or any launch with at least a workgroup per CU): one workgroup = one query row x 64 heads over its slots, so
-// each gathered row serves 64 heads.
+// Sparse MLA attention over many query rows for gfx950 (the arithmetic of dsa_attention.hip, for a prefill chunk's queries
+// and batches of decode rows: attention_wide_splits below has the rule): one workgroup = one query row, or one split of
+// its slots, x 64 heads, so each gathered row serves 64 heads; with splits combine_splits_kernel follows.
 //
 // What bounds it: both products on v_mfma_f32_32x32x16_bf16 are 68 products of 32 cycles per chunk of 64 slots and
 // SIMD (2,176 cycles), with e4m3 -> bf16 conversions of the keys (144 per wave) and the values (64). A wave issues at

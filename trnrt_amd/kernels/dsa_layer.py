@@ -114,8 +114,8 @@ class PooledDecodeLayer:
     """Buffers and launch parameters of a pooled (GLM, kpool kp > 1) decode step over B rows with up to max_pages
     pages each: the pooled indexer over the bf16 pool-key cache, the exact top-keep pools, sparse MLA over their
     tokens and the tail (trnrt/models/mla.py:505-526 `attention_long` for a decode batch), enqueued by one call of the
-    C ABI's dsa_pooled_decode_layer: one kernel launch per 8 rows where the shapes allow (512-wide rows, at most 32
-    indexer heads, rows of at most 8,192 pools), the separate kernels otherwise or with chain=True. Nothing is
+    C ABI's dsa_pooled_decode_layer: up to 16 rows in one kernel launch per 8 where the shapes allow (512-wide rows, at
+    most 32 indexer heads, rows of at most 8,192 pools), the separate kernels otherwise or with chain=True. Nothing is
     allocated per step.
 
     B, Hi (indexer heads), H (query heads), dqk (512: GLM's NoPE latent, or 576), max_pages, page_size, num_pages
