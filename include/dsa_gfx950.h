@@ -295,8 +295,9 @@ int dsa_decode_layer_chain(const void* q_idx_bf16, const float* w, const uint8_t
  * previous call's gets the difference filled on `stream` first, so calls of any batch sizes follow each other). A
  * call that cannot run in that size returns DSA_ESCRATCH before any HIP call. dsa_workspace_bytes(DSA_WS_LAYER, B, H,
  * keep, max_len, splits) of at most that size always runs; a batch whose query is larger may too, with fewer attention
- * splits than in a workspace of the queried size. Every call on a GPU shares that GPU's scratch: calls that overlap on one GPU (several streams, host
- * threads) race and must be serialised by the caller. Arguments and results as dsa_decode_layer.
+ * splits than in a workspace of the queried size. Every call on a GPU shares that GPU's scratch: calls that overlap on
+ * one GPU (several streams, host threads) race and must be serialised by the caller. Arguments and results as
+ * dsa_decode_layer.
  */
 #define DSA_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
 int dsa_decode_layer_noalloc(const void* q_idx_bf16, const float* w, const uint8_t* k_fp8, const float* k_scale,

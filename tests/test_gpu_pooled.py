@@ -101,9 +101,9 @@ def test_attend_pooled_tails_vs_oracle(kp, dqk, splits):
 ])
 def test_attend_pooled_many_row_form_in_its_workspace(B, H, kp, keep, dqk, form):
     """attend_pooled with 9 workgroups' rows and more (the many-row form in splits or one, or the split form), in a
-    workspace of exactly dsa_sparse_mla_pooled_workspace_bytes: every tail length, a row with no complete pool, fewer selected pools than
-    keep. The cache rows that no row attends are NaN (bytes and scale), the tokens of the tail's pool past the position
-    among them: a context's last pages hold such rows until they are written."""
+    workspace of exactly dsa_sparse_mla_pooled_workspace_bytes: every tail length, a row with no complete pool, fewer
+    selected pools than keep. The cache rows that no row attends are NaN (bytes and scale), the tokens of the tail's pool
+    past the position among them: a context's last pages hold such rows until they are written."""
     from trnrt_amd import _lib
     say(f"attend_pooled many-row form B={B} H={H} kp={kp} keep={keep} dqk={dqk}")
     g = torch.Generator().manual_seed(1000 * B + kp)

@@ -467,7 +467,8 @@ __global__ __launch_bounds__(128) void combine_splits_kernel(const float* __rest
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const float wt = (s < splits && ml[s].y > 0.0f) ? ml[s].y * (MANY ? __builtin_amdgcn_exp2f(ml[s].x - M) : __expf(ml[s].x - M)) : 0.0f;
+    const float dm = ml[s].x - M;  // (MANY: base 2)
+    const float wt = (s < splits && ml[s].y > 0.0f) ? ml[s].y * (MANY ? __builtin_amdgcn_exp2f(dm) : __expf(dm)) : 0.0f;
     W += wt;
     acc.x += wt * v[s].x;
     acc.y += wt * v[s].y;
